@@ -96,7 +96,7 @@ def draw(rng: random.Random) -> dict:
 def _transport(case: dict, k: int = 0) -> Task:
     """The k-th transport instance of a case: the first as stated, the next ones a quarter smaller each."""
     cut = lambda v, least: max(least, v * (4 - k) // 4)  # noqa: E731
-    return Task.from_text(gen.transport(cut(case["locations"], 4), cut(case["trucks"], 1), cut(case["packages"], 2),
+    return Task.from_text(gen.transport(cut(case["locations"], 6), cut(case["trucks"], 1), cut(case["packages"], 2),
                                         goals=min(32, cut(case["packages"], 2)), seed=k))
 
 
