@@ -1171,9 +1171,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     if (o.fingerprint)
     {
         set_small(kFingerprint, 0);
-        hipLaunchKernelGGL(k_fingerprint, dim3(std::min<u64>(blocks_for(set.size, 256), 2048)), dim3(256), 0, stream, set.v.arena,
-                           set.size, static_cast<u32>(W), d_slot_cid, small + kFingerprint);
-        launch_check("fingerprint");
+        launch_fingerprint(set.v.arena, set.size, W, d_slot_cid, task.slot_cid.size(), small + kFingerprint, stream);
         sync_small();
         r.fingerprint = b.host[kFingerprint];
     }

@@ -605,9 +605,7 @@ BrfsResultC brfs_wide(const CompiledTask& task, const TaskDev& dev, const BrfsOp
             d_slot_cid = c;
         }
         set_small(kFingerprint, 0);
-        hipLaunchKernelGGL(k_fingerprint, dim3(std::min<u64>(blocks_for(set.size, 256), 2048)), dim3(256), 0, stream, set.v.arena,
-                           set.size, W, d_slot_cid, small + kFingerprint);
-        launch_check("fingerprint");
+        launch_fingerprint(set.v.arena, set.size, W, d_slot_cid, task.slot_cid.size(), small + kFingerprint, stream);
         sync_small();
         r.fingerprint = b.host[kFingerprint];
     }
