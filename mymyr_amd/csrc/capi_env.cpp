@@ -24,7 +24,6 @@ struct EnvInstance
     TaskDev T{};
     u32 init_count = 0;
     u32 init_goal = 0;
-    u32 variant = 0;
 };
 
 struct mya_env
@@ -45,21 +44,8 @@ struct mya_env
     SamplerDev sampler{};          // the instance sampler (instances 0: off)
     u32* d_thresholds = nullptr;   // device [m - 1]
     i32* d_indices = nullptr;      // device [m]
-    // grouped launches: per variant present, its block shape
-    struct Launch
-    {
-        u32 variant;
-        unsigned nw;
-        size_t lds;
-        u32 wave_words;
-    };
-    std::vector<Launch> launches;
-    // the row groups of the last grouped call (device scratch, grown to the largest batch)
-    u64 group_rows = 0;
-    u32* d_hist = nullptr;   // [instances + 1]
-    u32* d_starts = nullptr;  // [instances + 1]
-    u32* d_chunks = nullptr;  // [instances + 1]
-    u32* d_order = nullptr;   // [group_rows]
+    u32 wave_words = 0;  // LDS words per wave of the env's launches
+    u32 general = 0;     // some instance is not simple
     u64 sampled_rows = 0;
     i32* d_sampled = nullptr;  // [sampled_rows]: the sampled next instances of a step
     std::mutex mutex;         // guards the scratch growth
@@ -111,10 +97,6 @@ VisitedDev visited_of(const mya_env_batch* b)
     return VisitedDev{b->visited, b->visited_count, b->visited_status, b->visited_capacity, b->visited_status_per_row ? 1u : 0u};
 }
 
-/// Whether a call runs grouped by instance: over several instances (a one-instance batch runs in batch order, checking
-/// its task ids on the way).
-bool grouped(const mya_env* e) { return e->instances() > 1; }
-
 /// The env's per-row scratch array `member` (of `have` rows), grown under the env's lock to `rows` (a call with a batch
 /// no larger than before allocates nothing).
 template<class X>
@@ -130,16 +112,6 @@ X* scratch_rows(mya_env* e, u64 rows, X* mya_env::*member, u64 mya_env::*have)
         e->*have = rows;
     }
     return e->*member;
-}
-
-/// Groups the batch's rows by instance into the env's scratch (grown under the env's lock; a call with a batch no
-/// larger than before allocates nothing).
-RowGroups group_rows(mya_env* e, const mya_env_batch* b, hipStream_t stream, u32* status = nullptr)
-{
-    scratch_rows(e, b->rows, &mya_env::d_order, &mya_env::group_rows);
-    launch_group_rows(b->task_ids, b->rows, e->instances(), e->d_hist, e->d_order, e->d_starts, e->d_chunks, status ? status : e->d_status,
-                      stream);
-    return RowGroups{e->d_order, e->d_starts, e->d_chunks};
 }
 
 /// The table's domain check (TaskTable::domain_mismatch, src/mymyr/rl/task_table.cpp:75-100): empty if `t` has the
@@ -165,7 +137,7 @@ std::string domain_mismatch(const TaskText& r, const TaskText& t)
     return {};
 }
 
-/// A count over the batch's rows (refresh, goal): in batch order over one instance, else grouped by instance.
+/// A count over the batch's rows (refresh, goal).
 void run_count(mya_env* env, const mya_env_batch* batch, CountArgs& a, hipStream_t s)
 {
     a.T = env->T0();
@@ -181,32 +153,15 @@ void run_count(mya_env* env, const mya_env_batch* batch, CountArgs& a, hipStream
     a.status = env->d_status;
     a.cache_width = env->cache_width();
     a.mask_width = env->num_schemas;
-    if (!grouped(env))
-    {
-        launch_env_count(a, s);
-        return;
-    }
-    a.groups = group_rows(env, batch, s);
-    if (env->instances() <= kPerInstanceLaunches)
-        for (u32 k = 0; k < env->instances(); ++k)
-        {
-            a.T = env->inst[k].T;
-            a.instance = k;
-            launch_env_count(a, s);
-        }
-    else
-        for (const mya_env::Launch& l : env->launches)
-        {
-            a.wave_words = l.wave_words;
-            launch_env_count_grouped(a, l.variant, l.nw, l.lds, s);
-        }
+    a.wave_words = env->wave_words;
+    a.general = env->general;
+    launch_env_count(a, s);
 }
 
 void free_env(mya_env* e)
 {
-    for (void* p : std::initializer_list<void*>{e->d_status, e->d_inst, e->d_tasks, e->d_init, e->d_init_cache, e->d_init_masks, e->d_hist,
-                                                e->d_starts, e->d_chunks, e->d_order, e->d_thresholds, e->d_indices,
-                                                e->d_sampled, e->d_seed})
+    for (void* p : std::initializer_list<void*>{e->d_status, e->d_inst, e->d_tasks, e->d_init, e->d_init_cache, e->d_init_masks, e->d_thresholds,
+                                                e->d_indices, e->d_sampled, e->d_seed})
         dev_free(p);
     if (e->h_status)
         (void)hipHostFree(e->h_status);
@@ -236,8 +191,7 @@ ExpandScratch carve_expand_scratch(void* block, u64 n)
     return x;
 }
 
-/// The flat expansion of rows over instances `inst` (one: batch order; several: grouped by instance with `env`'s
-/// scratch and the rows' task ids). `block` (device, at least expand_scratch_bytes(max(rows, 1)) bytes) holds the
+/// The flat expansion of rows over instances `inst` (several: `env`'s, with the rows' task ids). `block` (device, at least expand_scratch_bytes(max(rows, 1)) bytes) holds the
 /// expansion's scratch; the call synchronizes the stream before it returns, so the block is free again then.
 void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const int32_t* task_ids, const uint64_t* states, uint64_t rows,
                  uint32_t words, const mya_expand_options* options, mya_expansion* out, hipStream_t stream, void* block, mya_task* lazy)
@@ -290,27 +244,12 @@ void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const in
         a.witness = options->witness_pruning && a.T.witness ? 1 : 0;
         if (inst.size() > 1)
         {
-            mya_env_batch b{};
-            b.states = const_cast<uint64_t*>(states);
-            b.rows = rows;
-            b.words = words;
-            b.task_ids = const_cast<int32_t*>(task_ids);
-            a.groups = group_rows(env, &b, stream, words_status + 1);
+            a.tasks = env->d_tasks;
+            a.task_ids = task_ids;
+            a.instances = env->instances();
+            a.wave_words = env->wave_words;
+            a.general = env->general;
         }
-        // one launch over the batch, or one per instance over its group
-        auto launch = [&](ExpandArgs& x) {
-            if (!x.groups.order)
-            {
-                launch_expand(x, stream);
-                return;
-            }
-            for (u32 k = 0; k < inst.size(); ++k)
-            {
-                x.T = *inst[k];
-                x.instance = k;
-                launch_expand(x, stream);
-            }
-        };
         a.states = states;
         a.rows = rows;
         a.words = words;
@@ -322,7 +261,7 @@ void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const in
         a.words_needed = words_status;
         a.status = words_status + 1;
         a.pass = 0;
-        launch(a);
+        launch_expand(a, stream);
         launch_exclusive_scan(counts, pre, rows, scratch, pre + rows, stream);
         if (a.drop_noops)
         {
@@ -368,7 +307,7 @@ void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const in
             a.succ_hash = out->succ_hash;
             a.noop = out->noop;
             a.index = out->index;
-            launch(a);
+            launch_expand(a, stream);
         }
         hip_check(hipMemcpyAsync(st, words_status, sizeof(st), hipMemcpyDeviceToHost, stream), "expand status");
         hip_check(hipStreamSynchronize(stream), "expand");
@@ -380,7 +319,7 @@ void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const in
                 throw std::logic_error("mymyr_amd: expand: an added atom without a slot was not recorded");
             a.T = *device_task(lazy).thost;
             launch_fill_u32(words_status, 2, 0, stream);
-            launch(a);
+            launch_expand(a, stream);
             hip_check(hipMemcpyAsync(st, words_status, sizeof(st), hipMemcpyDeviceToHost, stream), "expand status");
             hip_check(hipStreamSynchronize(stream), "expand");
         }
@@ -436,10 +375,16 @@ void create_env(mya_task* const* tasks, uint32_t count, const mya_env_config* co
             EnvInstance& in = e->inst[i];
             in.task = tasks[i];
             in.T = *device_task(tasks[i]).thost;
-            in.variant = env_variant(in.T);
             e->words = std::max(e->words, in.T.W);
             e->label_width = std::max(e->label_width, in.T.label_width);
             e->num_schemas = std::max(e->num_schemas, in.T.num_schemas);
+            e->general |= in.T.simple ? 0u : 1u;
+        }
+        {
+            std::vector<const TaskDev*> all;
+            for (const EnvInstance& in : e->inst)
+                all.push_back(&in.T);
+            e->wave_words = env_wave_words(all.data(), count);
         }
         const u32 S = e->num_schemas, cw = e->cache_width();
         e->d_status = dev_alloc<u32>(1, "env status");
@@ -499,7 +444,6 @@ void create_env(mya_task* const* tasks, uint32_t count, const mya_env_config* co
             d.init_count = in.init_count;
             d.init_goal = in.init_goal;
             d.fluent_slots = in.T.fluent_slots;
-            d.variant = in.variant;
             d.init_hash = hash_state(tasks[i]->compiled->initial.data(), in.T.W);
             ht[i] = in.T;
         }
@@ -507,24 +451,6 @@ void create_env(mya_task* const* tasks, uint32_t count, const mya_env_config* co
         hip_check(hipMemcpy(e->d_inst, hi.data(), count * sizeof(InstDev), hipMemcpyHostToDevice), "env instances");
         e->d_tasks = dev_alloc<TaskDev>(count, "env instance tables");
         hip_check(hipMemcpy(e->d_tasks, ht.data(), count * sizeof(TaskDev), hipMemcpyHostToDevice), "env instance tables");
-        if (count > 1)
-        {
-            for (u32 v = 0; v < 4; ++v)
-            {
-                std::vector<const TaskDev*> of;
-                for (const EnvInstance& in : e->inst)
-                    if (in.variant == v)
-                        of.push_back(&in.T);
-                if (of.empty())
-                    continue;
-                mya_env::Launch l{v, 0, 0, 0};
-                l.nw = grouped_shape(of.data(), static_cast<u32>(of.size()), &l.lds, &l.wave_words);
-                e->launches.push_back(l);
-            }
-            e->d_hist = dev_alloc<u32>(count + 1, "env group counters");
-            e->d_starts = dev_alloc<u32>(count + 1, "env group starts");
-            e->d_chunks = dev_alloc<u32>(count + 1, "env group chunks");
-        }
         *out = e.release();
     }
 }
@@ -716,28 +642,15 @@ void env_step(mya_env* env, const mya_env_batch* batch, const mya_step_outputs* 
             launch_env_sample_next(env->sampler, env->d_seed, batch->first_env, batch->rows, batch->reset_counts, batch->sampling_seeds,
                                    batch->env_ids, const_cast<i32*>(a.next_task_ids), s);
         }
-        if (!grouped(env))
+        a.wave_words = env->wave_words;
+        a.general = env->general;
+        if (a.instances == 1)
         {
-            // the batch-order step runs every row as instance 0: given ids are only checked
+            // every row runs as instance 0: given ids are only checked
             launch_check_ids(batch->task_ids, batch->rows, 1, env->d_status, s);
             launch_check_ids(next_task_ids, batch->rows, 1, env->d_status, s);
-            launch_env_step(a, s);
-            return;
         }
-        a.groups = group_rows(env, batch, s);
-        if (env->instances() <= kPerInstanceLaunches)
-            for (u32 k = 0; k < env->instances(); ++k)
-            {
-                a.T = env->inst[k].T;
-                a.instance = k;
-                launch_env_step(a, s);
-            }
-        else
-            for (const mya_env::Launch& l : env->launches)
-            {
-                a.wave_words = l.wave_words;
-                launch_env_step_grouped(a, l.variant, l.nw, l.lds, s);
-            }
+        launch_env_step(a, s);
     }
 }
 }  // namespace
@@ -787,12 +700,7 @@ int mya_env_reserve(mya_env* env, uint64_t rows)
         if (rows == 0)
             return;
         scratch_rows(env, rows, &mya_env::d_sampled, &mya_env::sampled_rows);
-        if (grouped(env))
-            scratch_rows(env, rows, &mya_env::d_order, &mya_env::group_rows);
-        for (const EnvInstance& in : env->inst)
-            prepare_env_launches(in.T);
-        for (const mya_env::Launch& l : env->launches)
-            prepare_grouped_launches(l.variant, l.lds);
+        prepare_env_launches(env->wave_words, env->general, env->instances() == 1);
     });
 }
 

@@ -32,8 +32,6 @@ struct InstDev
     u32 init_count;
     u32 init_goal;
     u32 fluent_slots;
-    u32 variant;  // the kernel variant that runs the instance's rows (staged | levels << 1)
-    u32 reserved;
     u64 init_hash;  // hash_state of the initial state (its visited-table key)
 };
 
@@ -48,15 +46,6 @@ struct VisitedDev
     u32 status_per_row;
 };
 
-/// Rows of a batch over several instances grouped by instance (a counting sort of the task ids): order lists the rows
-/// of instance 0, then of instance 1, ...; instance k's rows are order[starts[k], starts[k + 1]), cut into chunks of
-/// kChunkRows rows numbered from chunk_start[k]. Rows whose task id names no instance are in no group.
-struct RowGroups
-{
-    const u32* order;
-    const u32* starts;       // [instances + 1]
-    const u32* chunk_start;  // [instances + 1]
-};
 /// An instance sampler on the device (rl/sampling.hpp): instances 0 is off; m 0 draws uniformly.
 struct SamplerDev
 {
@@ -66,18 +55,16 @@ struct SamplerDev
     const i32* indices;     // [m]
 };
 
-constexpr u32 kChunkRows = 4;  // rows of a chunk: one block's share (one per wave of a block of 4 waves)
 constexpr u32 kMaxInstances = 65536;
 
 struct EnvArgs
 {
-    TaskDev T;             // the instance of a one-instance batch
-    const TaskDev* tasks;  // [instances] (device): every instance's tables, for a grouped launch
+    TaskDev T;             // the instance of a one-instance env
+    const TaskDev* tasks;  // [instances] (device): every instance's tables
     const InstDev* inst;   // [instances] (device)
     u32 instances;
-    u32 wave_words;        // LDS words per wave of a grouped launch (the largest of its instances)
-    RowGroups groups;      // rows grouped by instance (order null: batch order, one instance)
-    u32 instance;          // with groups, a one-instance launch's instance (T's): it steps that group's rows
+    u32 wave_words;        // LDS words per wave (the largest of the instances; 0: T's)
+    u32 general;           // some instance is not simple (one instance: T tells)
     EnvCfg cfg;
     u64* states;
     u64 rows;
@@ -146,7 +133,7 @@ struct CountArgs
     const InstDev* inst;
     u32 instances;
     u32 wave_words;
-    RowGroups groups;
+    u32 general;
     const u64* states;
     u64 rows;
     u32 words;
@@ -160,7 +147,7 @@ struct CountArgs
     const u64* goal_pos;
     const u64* goal_neg;
     u32* status;
-    u32 instance;  // the instance of a one-instance count (its fingerprint salt; with groups, the group it counts)
+    u32 instance;  // the instance of a one-instance count (its fingerprint salt)
 };
 
 void launch_env_count(const CountArgs& a, hipStream_t stream);
@@ -170,27 +157,11 @@ void launch_env_count(const TaskDev& T, const u64* states, u64 rows, u32 words, 
                       hipStream_t stream, const u64* goal_pos = nullptr, const u64* goal_neg = nullptr, u32* status = nullptr,
                       u32 instance = 0, u32 schemas = 0);
 
-/// Groups the rows by task id (RowGroups): hist [instances + 1] and the three group arrays are device scratch; rows
-/// with a task id outside [0, instances) set kStatusTaskId.
-void launch_group_rows(const i32* task_ids, u64 rows, u32 instances, u32* hist, u32* order, u32* starts, u32* chunk_start,
-                       u32* status, hipStream_t stream);
-
-/// Tables of at most this many instances step with one launch per instance (the instance's tables as kernel arguments,
-/// its group's rows from the row groups); larger tables with one launch per kernel variant (each block reads its
-/// chunk's instance's tables from device memory).
-constexpr u32 kPerInstanceLaunches = 16;
-
-/// The kernel variant of an instance (InstDev::variant) and the block shape of a grouped launch over the instances of
-/// one variant: waves per block and dynamic LDS bytes, from the largest hot tables and per-wave region among them.
-u32 env_variant(const TaskDev& T);
-unsigned grouped_shape(const TaskDev* const* tasks, u32 n, size_t* lds_bytes, u32* wave_words);
-/// Raises the dynamic LDS limits of the step and count kernels an instance (or a variant's grouped launch) uses, so
-/// that later launches make no runtime call besides the launch (HIP graph capture).
-void prepare_env_launches(const TaskDev& T);
-void prepare_grouped_launches(u32 v, size_t lds);
-/// The grouped step / count of the rows of the instances of variant v (grid: enough blocks for every chunk).
-void launch_env_step_grouped(const EnvArgs& a, u32 v, unsigned nw, size_t lds, hipStream_t stream);
-void launch_env_count_grouped(const CountArgs& a, u32 v, unsigned nw, size_t lds, hipStream_t stream);
+/// The LDS words per wave of launches over the instances (their largest); throws for an instance the kernels cannot take.
+u32 env_wave_words(const TaskDev* const* tasks, u32 n);
+/// Raises the dynamic LDS limits of the step and count kernels of an env of one instance (`one`) or several, so that later
+/// launches make no runtime call besides the launch (HIP graph capture).
+void prepare_env_launches(u32 wave_words, bool general, bool one);
 
 /// Ascending true-atom slots of each row, -1 padded to max_atoms (State::slots, include/mymyr/state/state.hpp:96-101).
 void launch_encode_atoms(const u64* states, u64 rows, u32 words, u32 W, i32* out, u32 max_atoms, u32* status, hipStream_t stream);
@@ -236,13 +207,16 @@ __host__ __device__ inline u32 cache_width(const TaskDev& T) { return T.num_sche
 
 /// The flat expansion of rows (rl::expand, include/mymyr/rl/expand.hpp:1-130). Pass 0 counts each row's successors
 /// (and, with drop_noops, its no-op successors) and checks that rows have no atoms past their instance's slots; pass 1
-/// writes the successors of row i from offsets[i] on (kept rows only with drop_noops), up to capacity. Over a table,
-/// one launch per instance expands that instance's group of rows.
+/// writes the successors of row i from offsets[i] on (kept rows only with drop_noops), up to capacity. Over a table
+/// every row is expanded with its own instance's tables.
 struct ExpandArgs
 {
     TaskDev T;
-    RowGroups groups;  // rows grouped by instance (order null: batch order, one instance)
-    u32 instance;      // with groups, the instance (T's) whose group this launch expands
+    const TaskDev* tasks;  // over a table: [instances] (device), row i's instance in task_ids[i] (null: T for every row)
+    const i32* task_ids;
+    u32 instances;
+    u32 wave_words;        // LDS words per wave (0: T's)
+    u32 general;           // some instance is not simple (one instance: T tells)
     const u64* states;
     u64 rows;
     u32 words;
@@ -270,6 +244,23 @@ struct ExpandArgs
 };
 
 void launch_expand(const ExpandArgs& a, hipStream_t stream);
+
+/// The kernels over the lifted matching, by what they take (env_device.hpp); step_plain may be null (step serves).
+struct EnvKernels
+{
+    void (*step_plain)(EnvArgs);
+    void (*step)(EnvArgs);
+    void (*step_visited)(EnvArgs);
+    void (*step_table)(EnvArgs);
+    void (*count)(CountArgs);
+    void (*count_table)(CountArgs);
+    void (*expand)(ExpandArgs);
+    void (*expand_witness)(ExpandArgs);
+    void (*expand_table)(ExpandArgs);
+    void (*successors)(TaskDev, const u64*, u64, u32, u32, i32*, i32*, i32*, u64*, u32*);
+};
+/// The kernels for any task.
+EnvKernels env_kernels_general();
 /// kept[i] = counts[i] - noops[i], or counts[i] when every successor of row i is a no-op.
 void launch_kept_counts(const u32* counts, const u32* noops, u64 rows, u32* kept, hipStream_t stream);
 

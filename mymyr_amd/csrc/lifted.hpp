@@ -11,9 +11,9 @@
 // The set of bindings is the reference's (all literals of the precondition hold; witness pruning off), and the
 // lexicographic order is its canonical order (include/mymyr/successor/successors.hpp:8-10, 154-248).
 //
-// A block stages the task's hot tables (schemas, plans, constraints, checks, effects, view pairs, slot decoding,
-// dom0, goal, per-predicate tables: the image's first hot_words words) in LDS once; each wave of the block then
-// steps its environments with its own LDS region (state row, view, bindings, enumeration cursors).
+// The plans are the same for every lane, so the kernels read them (schemas, steps, terms, checks) through the constant
+// address space with wave-uniform indices: scalar loads and scalar branches, while the vector units do only the
+// candidates' bit work. Each wave has its own LDS region (state row, view, lane bindings).
 
 #include "device_common.hpp"
 #include "scan.hpp"
@@ -21,27 +21,25 @@
 
 namespace mya
 {
-/// The task as the kernels see it: hot sections by word offset (in the image and, once staged, in LDS), cold tables
-/// by global pointer.
+/// The task as the kernels see it: sections by word offset in the image, tables read lane by lane by pointer.
 struct TaskDev
 {
-    u64 off_schemas, off_steps, off_cons, off_checks, off_effects, off_pairs, off_decode, off_dom0;
+    u64 off_schemas, off_deltas, off_checks, off_effects, off_pairs, off_decode;
     u64 off_goal_pos, off_goal_neg, off_pred_arity, off_pos_begin, off_pred_pairs, off_pred_offset;
     const u64* image;
     const u64* rs;
     const u32* slot_of;
     const u64* records;
-    const u64* static_rows;
     const DevStaticMeta* static_meta;
     const u64* static_words;  // image base (static keys are image offsets)
     const u64* initial;
     u64 fluent_count;
-    u32 hot_words;
     u32 n, ow, W, num_schemas, num_pairs, view_words, ngp, ngn, goal_unsat, dense, label_width, fluent_slots;
     u32 num_decode, decode_arith;
-    u32 max_step_words;
+    u32 simple;    // no literal is checked one by one and no schema has more than kLaneDepth + 1 parameters
     u32 lazy;      // lazy slots: an added atom without a slot is recorded in `missing`
     u64* missing;  // lazy slots: bit per canonical fluent atom (device; set by the successor kernels), else null
+    u32 l_row, l_dfs_m, l_ub, l_bind, l_counts, l_dfs_w, l_eff, l_before, l_cur, l_words;  // a wave's LDS region (set_region)
     const DevWitness* witness;  // per schema its witness parameters and plans (null: no schema has a witness)
 };
 
@@ -49,20 +47,29 @@ struct TaskDev
 TaskDev task_dev(const u64* image_dev, const DevTaskHeader& h);
 
 constexpr u32 kMaxEnvSchemas = 8192;  // schemas whose per-state counts a wave keeps in LDS
-constexpr u32 kCap = 64;           // items per level of the level-synchronous count (one per lane)
+constexpr u32 kMaxEff = 32;        // effects per schema the step applies (more set kStatusCapacity)
 
-/// Per-wave LDS words: the state row, the view, the uniform binding, the bindings and per-level enumeration cursors of
-/// the 64 lanes' nested loops (A = the largest schema arity, at least 1), the effect scratch, the per-schema counts and
-/// the successor enumeration's level cursors (A masks, A words);
-/// with `levels`, also the two item levels of the level-synchronous count with their roots, root counts, root objects
-/// and item makers.
-__host__ __device__ inline u32 wave_lds_words(const TaskDev& t, bool levels)
+/// The word offsets of a wave's LDS region: the view, the state row, then the uniform binding, the 64 lanes' bindings
+/// (A = the largest schema arity, at least 1), the per-schema counts, the successor enumeration's level cursors (A
+/// masks, A words), the effect scratch, and for plans deeper than kLaneDepth the lanes' enumeration cursors.
+inline void set_region(TaskDev& t)
 {
     const u32 A = t.label_width ? t.label_width : 1;
-    const u32 S = t.num_schemas;
-    u32 w = t.W + t.view_words + (A + 1) / 2 + 32 * A + 64 * A + 32 * A + 32 + (S + 1) / 2 + A + (A + 1) / 2;
-    if (levels)
-        w += kCap * A + 5 * kCap / 2;
-    return (w + 1) & ~1u;
+    u32 w = t.view_words;
+    auto next = [&](u32 words) {
+        const u32 at = w;
+        w += words;
+        return at;
+    };
+    t.l_row = next(t.W);
+    t.l_dfs_m = next(A);
+    t.l_ub = next((A + 1) / 2);
+    t.l_bind = next(32 * A);
+    t.l_counts = next((t.num_schemas + 1) / 2);
+    t.l_dfs_w = next((A + 1) / 2);
+    t.l_eff = next(kMaxEff / 2);
+    t.l_before = next(kMaxEff / 2);
+    t.l_cur = next(A > kLaneDepth ? 64 * A + 32 * A : 0);
+    t.l_words = (w + 2) & ~1u;  // a word past the end: reads of two words at a bit position stay inside
 }
 }  // namespace mya

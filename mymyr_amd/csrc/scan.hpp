@@ -10,17 +10,24 @@ constexpr int kWave = 64;
 
 __device__ __forceinline__ u32 lane_id() { return __lane_id(); }
 
-/// Inclusive prefix sum across the 64 lanes of a wave.
+/// v moved across lanes by a DPP control (0 where no lane or a masked row feeds one): register moves, where a shuffle is
+/// a trip through the LDS unit of about a hundred cycles per step.
+template<int kCtrl, int kRows>
+__device__ __forceinline__ u32 dpp_move(u32 v)
+{
+    return static_cast<u32>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), kCtrl, kRows, 0xF, false));
+}
+
+/// Inclusive prefix sum across the 64 lanes of a wave (every lane active): within rows of 16 lanes by row shifts, then
+/// the rows' last lanes broadcast to the rows after them.
 __device__ __forceinline__ u32 wave_inclusive(u32 v)
 {
-    const u32 lane = lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1)
-    {
-        const u32 t = __shfl_up(v, d, kWave);
-        if (lane >= static_cast<u32>(d))
-            v += t;
-    }
+    v += dpp_move<0x111, 0xF>(v);
+    v += dpp_move<0x112, 0xF>(v);
+    v += dpp_move<0x114, 0xF>(v);
+    v += dpp_move<0x118, 0xF>(v);
+    v += dpp_move<0x142, 0xA>(v);
+    v += dpp_move<0x143, 0xC>(v);
     return v;
 }
 
@@ -37,20 +44,25 @@ __device__ __forceinline__ u64 wave_inclusive64(u64 v)
     return v;
 }
 
-__device__ __forceinline__ u32 wave_sum(u32 v)
+/// Lane k's value in every lane (k the same in every lane).
+__device__ __forceinline__ u32 lane_value(u32 v, u32 k) { return static_cast<u32>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(k))); }
+__device__ __forceinline__ u64 lane_value(u64 v, u32 k)
 {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1)
-        v += __shfl_xor(v, d, kWave);
-    return v;
+    return static_cast<u64>(lane_value(static_cast<u32>(v), k)) | (static_cast<u64>(lane_value(static_cast<u32>(v >> 32), k)) << 32);
 }
+
+__device__ __forceinline__ u32 wave_sum(u32 v) { return lane_value(wave_inclusive(v), kWave - 1); }
 
 __device__ __forceinline__ u64 wave_sum64(u64 v)
 {
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1)
-        v += __shfl_xor(v, d, kWave);
-    return v;
+    auto add = [&](u32 lo, u32 hi) { v += static_cast<u64>(lo) | (static_cast<u64>(hi) << 32); };
+    add(dpp_move<0x111, 0xF>(static_cast<u32>(v)), dpp_move<0x111, 0xF>(static_cast<u32>(v >> 32)));
+    add(dpp_move<0x112, 0xF>(static_cast<u32>(v)), dpp_move<0x112, 0xF>(static_cast<u32>(v >> 32)));
+    add(dpp_move<0x114, 0xF>(static_cast<u32>(v)), dpp_move<0x114, 0xF>(static_cast<u32>(v >> 32)));
+    add(dpp_move<0x118, 0xF>(static_cast<u32>(v)), dpp_move<0x118, 0xF>(static_cast<u32>(v >> 32)));
+    add(dpp_move<0x142, 0xA>(static_cast<u32>(v)), dpp_move<0x142, 0xA>(static_cast<u32>(v >> 32)));
+    add(dpp_move<0x143, 0xC>(static_cast<u32>(v)), dpp_move<0x143, 0xC>(static_cast<u32>(v >> 32)));
+    return lane_value(v, kWave - 1);
 }
 
 /// Exclusive prefix of v over a block of BLOCK threads; *total receives the block sum. Uses BLOCK/64 words of LDS.

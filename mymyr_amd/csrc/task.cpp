@@ -1212,7 +1212,12 @@ private:
         std::vector<DevCons> cons;
         std::vector<DevCheck> checks;
         std::vector<DevEffect> effects;
+        std::vector<DevDelta> deltas;
+        std::vector<u32> step_schema;  // per step: its schema
         std::vector<u64> dom0_words;
+        // per schema: makes a step, and pushes the count plan of the unbound parameters
+        std::vector<std::function<DevStep(u32, const std::vector<u8>&)>> step_makers;
+        std::vector<std::function<void(std::vector<u8>)>> plan_makers;
         // static k-ary relations used by checks
         std::map<u32, u32> static_rel;  // pred -> index
         std::vector<DevStaticMeta> static_meta;
@@ -1272,7 +1277,7 @@ private:
             ds.ground_end = static_cast<u32>(checks.size());
 
             // a step binding `v` after the parameters marked in `bound`
-            auto make_step = [&](u32 v, const std::vector<u8>& bound)
+            auto make_step = [this, &cons, &checks, &rel_of, &s, lo, wwords, dom_off, si](u32 v, const std::vector<u8>& bound)
             {
                 DevStep st{};
                 st.param = v;
@@ -1330,14 +1335,10 @@ private:
                 return st;
             };
 
-            // plans P_j: parameters [0, j) bound, the rest in greedy order
-            for (u32 j = 0; j <= s.arity; ++j)
+            // the count plan of the parameters not in `bound`, in greedy order
+            auto make_plan = [this, &steps, &s, make_step, si](std::vector<u8> bound)
             {
-                ds.plan_begin[j] = static_cast<u32>(steps.size());
-                std::vector<u8> bound(s.arity, 0);
-                for (u32 v = 0; v < j; ++v)
-                    bound[v] = 1;
-                for (u32 placed = j; placed < s.arity; ++placed)
+                for (u32 left = static_cast<u32>(std::count(bound.begin(), bound.end(), u8{0})); left; --left)
                 {
                     int best = -1;
                     long best_score = 0;
@@ -1365,6 +1366,17 @@ private:
                     steps.push_back(make_step(static_cast<u32>(best), bound));
                     bound[best] = 1;
                 }
+            };
+            step_makers.push_back(make_step);
+            plan_makers.push_back(make_plan);
+            // plans P_j: parameters [0, j) bound
+            for (u32 j = 0; j <= s.arity; ++j)
+            {
+                ds.plan_begin[j] = static_cast<u32>(steps.size());
+                std::vector<u8> bound(s.arity, 0);
+                for (u32 v = 0; v < j; ++v)
+                    bound[v] = 1;
+                make_plan(bound);
             }
             ds.plan_begin[s.arity + 1] = static_cast<u32>(steps.size());
             for (u32 j = s.arity + 2; j < kMaxParams + 2; ++j)
@@ -1419,6 +1431,8 @@ private:
                     for (u32 i = 0; i < l.terms.size(); ++i)
                     {
                         const u32 pos = C->layout.pos_begin[l.pred] + i;
+                        if (i < 2)
+                            e.terms[i] = l.terms[i];
                         if (l.terms[i] < 0)
                             e.base += C->layout.rs[pos][term_object(l.terms[i])];
                         else
@@ -1435,11 +1449,14 @@ private:
             for (const Literal& l : s.eff)
                 ds.nadd += l.positive ? 1 : 0;
             schemas.push_back(ds);
+            step_schema.resize(steps.size(), si);
         }
-        // which schemas' successor counts an action of schema a can change: an add or delete effect of a that can be an
-        // atom of a fluent precondition literal of s (the same predicate, and at every position the two terms can take
-        // a common object: a constant, or a parameter's static domain); a schema no action of a can touch keeps its
-        // count across the move. With more than 32 schemas every schema counts as changed.
+        // How an action of schema a changes the successor count of schema s: through the effects of a that can be an atom of
+        // a fluent precondition literal of s (the same predicate, and at every position the two terms can take a common
+        // object: a constant, or a parameter's static domain). No such effect: the count stays. Where the effects of one
+        // sign meet at most one literal of s, a positive one, the bindings lost are those of the state whose literal is
+        // a deleted atom and the bindings gained those of the reached state whose literal is an added atom (DevDelta);
+        // otherwise, and with more than 32 schemas, s is counted again.
         {
             const u32 S = static_cast<u32>(schemas.size());
             auto dom_of = [&](u32 si, i32 t) {
@@ -1456,26 +1473,137 @@ private:
                         return true;
                 return false;
             };
+            auto inside = [](const Bits& x, const Bits& y) {
+                for (size_t w = 0; w < x.size(); ++w)
+                    if (x[w] & ~y[w])
+                        return false;
+                return true;
+            };
+            struct Match
+            {
+                u32 effect, lit;  // effect: position in the device's effect list (adds, then deletes)
+                const Literal* e;
+            };
+            // the DevDelta of schema s for effect m of schema a (false: none of this form)
+            auto make_delta = [&](u32 a, u32 s2, const Match& m, DevDelta& d) {
+                const Literal& l = T->schemas[s2].pre[m.lit];
+                if (l.terms.size() > kMaxDeltaTerms)
+                    return false;
+                d = DevDelta{};
+                d.schema = s2;
+                d.effect = m.effect;
+                std::vector<u8> bound(T->schemas[s2].arity, 0);
+                for (size_t i = 0; i < l.terms.size(); ++i)
+                {
+                    const i32 lt = l.terms[i], et = m.e->terms[i];
+                    i32 other = lt;  // what et must equal: the literal's constant, or the term its parameter already took
+                    if (lt >= 0)
+                    {
+                        u32 k = 0;
+                        while (k < d.nbound && d.param[k] != lt)
+                            ++k;
+                        if (k == d.nbound)
+                        {
+                            d.param[k] = lt;
+                            d.term[k] = et;
+                            ++d.nbound;
+                            if (!inside(dom_of(a, et), C->dom0[s2][static_cast<u32>(lt)]))
+                                d.tests = 1;
+                            continue;
+                        }
+                        other = d.term[k];
+                    }
+                    if (et == other)
+                        continue;
+                    d.eq[2 * d.neq] = et;
+                    d.eq[2 * d.neq + 1] = other;
+                    ++d.neq;
+                }
+                for (u32 k = 0; k < d.nbound; ++k)
+                    bound[static_cast<u32>(d.param[k])] = 1;
+                for (size_t j = 0; j < T->schemas[s2].pre.size(); ++j)
+                {
+                    const Literal& x = T->schemas[s2].pre[j];
+                    const auto ps = distinct_params(x.terms);
+                    bool all = j != m.lit && !ps.empty() && !(T->preds[x.pred].kind == 'S' && T->preds[x.pred].arity == 1);
+                    for (u32 q : ps)
+                        all = all && bound[q];
+                    if (all)
+                        d.tests = 1;
+                }
+                d.test_begin = static_cast<u32>(steps.size());
+                if (d.tests)
+                {
+                    std::vector<u8> b2(bound.size(), 0);
+                    for (u32 k = 0; k < d.nbound; ++k)
+                    {
+                        steps.push_back(step_makers[s2](static_cast<u32>(d.param[k]), b2));
+                        b2[static_cast<u32>(d.param[k])] = 1;
+                    }
+                }
+                d.plan_begin = static_cast<u32>(steps.size());
+                plan_makers[s2](bound);
+                d.plan_end = static_cast<u32>(steps.size());
+                step_schema.resize(steps.size(), s2);
+                return true;
+            };
             for (u32 a = 0; a < S; ++a)
             {
-                u32 mask = S > 32 ? ~0u : 0u;
+                DevSchema& ds = schemas[a];
+                ds.recount = S > 32 ? ~0u : 0u;
+                std::vector<DevDelta> dels, adds;
                 for (u32 s2 = 0; s2 < S && S <= 32; ++s2)
                 {
-                    bool hit = false;
-                    for (const Literal& e : T->schemas[a].eff)
-                        for (const Literal& l : T->schemas[s2].pre)
+                    if (schemas[s2].never)
+                        continue;
+                    std::vector<Match> matches;
+                    std::set<u32> lits[2];
+                    bool plain = schemas[s2].ground_begin == schemas[s2].ground_end;
+                    for (int pass = 0, e = 0; pass < 2; ++pass)
+                        for (const Literal& el : T->schemas[a].eff)
                         {
-                            if (hit || l.pred != e.pred || T->preds[l.pred].kind != 'F' || l.terms.size() != e.terms.size())
+                            if (el.positive != (pass == 0))
                                 continue;
-                            bool all = true;
-                            for (size_t i = 0; i < l.terms.size() && all; ++i)
-                                all = meet(dom_of(a, e.terms[i]), dom_of(s2, l.terms[i]));
-                            hit = all;
+                            for (u32 j = 0; j < T->schemas[s2].pre.size(); ++j)
+                            {
+                                const Literal& l = T->schemas[s2].pre[j];
+                                if (l.pred != el.pred || T->preds[l.pred].kind != 'F' || l.terms.size() != el.terms.size())
+                                    continue;
+                                bool all = true;
+                                for (size_t i = 0; i < l.terms.size() && all; ++i)
+                                    all = meet(dom_of(a, el.terms[i]), dom_of(s2, l.terms[i]));
+                                if (!all)
+                                    continue;
+                                plain = plain && l.positive && e < 32;
+                                lits[pass].insert(j);
+                                matches.push_back(Match{static_cast<u32>(e), j, &el});
+                            }
+                            ++e;
                         }
-                    if (hit)
-                        mask |= 1u << s2;
+                    if (matches.empty())
+                        continue;
+                    plain = plain && lits[0].size() <= 1 && lits[1].size() <= 1 && matches.size() <= 8;
+                    std::vector<DevDelta> mine;
+                    for (const Match& m : matches)
+                    {
+                        DevDelta d;
+                        plain = plain && make_delta(a, s2, m, d);
+                        if (plain)
+                            mine.push_back(d);
+                    }
+                    if (!plain)
+                    {
+                        ds.recount |= 1u << s2;
+                        continue;
+                    }
+                    for (const DevDelta& d : mine)
+                        (d.effect < ds.nadd ? adds : dels).push_back(d);
                 }
-                schemas[a].affects = mask;
+                ds.del_begin = static_cast<u32>(deltas.size());
+                deltas.insert(deltas.end(), dels.begin(), dels.end());
+                ds.add_begin = static_cast<u32>(deltas.size());
+                deltas.insert(deltas.end(), adds.begin(), adds.end());
+                ds.add_end = static_cast<u32>(deltas.size());
             }
         }
 
@@ -1520,6 +1648,116 @@ private:
                 view_words += p.src_n * p.dst_words;
             pairs.push_back(p);
         }
+        // the terms of the steps' constraints, resolved against the pairs and the steps' windows
+        std::vector<DevTerm> terms(cons.size());
+        std::vector<u64> term_rows;
+        std::vector<u8> static_term(cons.size(), 0);  // Image terms over term_rows (the others: over the dom0 bits)
+        {
+            std::map<std::array<u32, 3>, u32> row_tables;  // (static row table, window start, words) -> first word
+            auto dom_bits = [&](u32 pred, u32 pos) {  // the objects an atom of `pred` can have at position `pos`
+                Bits b(ow, 0);
+                for (u32 o : C->layout.domain[C->layout.pos_begin[pred] + pos])
+                    set_bit(b, o);
+                return b;
+            };
+            for (u32 k = 0; k < steps.size(); ++k)
+            {
+                DevStep& st = steps[k];
+                const auto& dom0 = C->dom0[step_schema[k]];
+                st.term_begin = st.cons_begin;
+                for (u32 ci = st.cons_begin; ci < st.cons_end; ++ci)
+                {
+                    const DevCons& c = cons[ci];
+                    DevTerm& t = terms[ci];
+                    t.neg = c.neg;
+                    t.src = kNone;
+                    t.rows = kNone;
+                    if (c.kind == static_cast<u32>(ConsKind::Dom0))
+                    {
+                        t.path = static_cast<u32>(TermPath::Image);
+                        t.base = c.table;
+                        continue;
+                    }
+                    Bits can(ow, 0);  // the objects the rows can hold
+                    if (c.kind == static_cast<u32>(ConsKind::StaticRow))
+                    {
+                        const std::vector<u64>& rows = m_row_data[c.table];
+                        for (u32 o = 0; o < n; ++o)
+                            for (u32 w = 0; w < ow; ++w)
+                                can[w] |= rows[static_cast<size_t>(o) * ow + w];
+                        const std::array<u32, 3> key{c.table, st.lo, st.words};
+                        auto it = row_tables.find(key);
+                        if (it == row_tables.end())
+                        {
+                            it = row_tables.emplace(key, static_cast<u32>(term_rows.size())).first;
+                            for (u32 o = 0; o < n; ++o)
+                                for (u32 w = 0; w < st.words; ++w)
+                                {
+                                    const u32 at = st.lo + 64 * w, sh = at & 63;
+                                    const u64* r = rows.data() + static_cast<size_t>(o) * ow;
+                                    u64 v = (at >> 6) < ow ? r[at >> 6] >> sh : 0;
+                                    if (sh && (at >> 6) + 1 < ow)
+                                        v |= r[(at >> 6) + 1] << (64 - sh);
+                                    term_rows.push_back(v);
+                                }
+                        }
+                        t.path = static_cast<u32>(TermPath::Image);
+                        static_term[ci] = 1;
+                        t.src = c.src;
+                        t.base = it->second;
+                        t.stride = st.words;
+                    }
+                    else
+                    {
+                        const DevPair& p = pairs[c.table];
+                        const bool unary = T->preds[p.pred].arity == 1;
+                        can = dom_bits(p.pred, unary ? 0 : (p.dir == 0 ? 1 : 0));
+                        const i64 delta = static_cast<i64>(st.lo) - static_cast<i64>(p.dst_lo);
+                        t.delta = static_cast<i32>(delta);
+                        if (c.kind == static_cast<u32>(ConsKind::ViewRow))
+                        {
+                            if (c.src == kNone)
+                            {
+                                t.row0 = c.obj - p.src_lo;
+                                if (t.row0 >= p.src_n)
+                                    t.rows = p.src_n;  // a constant outside the rows: no candidate
+                            }
+                            else
+                            {
+                                t.src = c.src;
+                                t.row0 = p.src_lo;
+                                for (u32 o = 0; o < n; ++o)
+                                    if (test_bit(dom0[c.src], o) && o - p.src_lo >= p.src_n)
+                                        t.rows = p.src_n;
+                            }
+                        }
+                        // the wave's region holds the view, then the state row
+                        const u64 bit0 = p.bulk ? 64 * static_cast<u64>(view_words) + p.bit0 : 64 * static_cast<u64>(p.offset);
+                        const u64 row_bits = p.bulk ? p.row_bits : 64 * static_cast<u64>(p.dst_words);
+                        if (bit0 + row_bits * p.src_n > 0xFFFFFFFFull)
+                            throw Error("the task's state and view exceed the device path's 32-bit bit offsets");
+                        if (row_bits % 64 == 0 && bit0 % 64 == 0 && delta >= 0 && delta % 64 == 0 && delta + 64 * static_cast<i64>(st.words) <= static_cast<i64>(row_bits))
+                        {
+                            t.path = static_cast<u32>(TermPath::Words);
+                            t.base = static_cast<u32>(bit0 / 64 + static_cast<u64>(delta) / 64);
+                            t.stride = static_cast<u32>(row_bits / 64);
+                        }
+                        else
+                        {
+                            t.path = static_cast<u32>(TermPath::Bits);
+                            t.base = static_cast<u32>(bit0);
+                            t.stride = static_cast<u32>(row_bits);
+                        }
+                    }
+                    // a positive term whose rows hold no object of the window outside the static domain implies dom0
+                    bool implied = !c.neg;
+                    for (u32 o = st.lo; o < n && o < st.lo + 64 * st.words && implied; ++o)
+                        implied = !test_bit(can, o) || test_bit(dom0[st.param], o);
+                    if (implied)
+                        st.term_begin = st.cons_begin + 1;
+                }
+            }
+        }
         // slot decoding per fluent predicate (ascending offset)
         std::vector<DevPredDecode> decode;
         bool decode_arith = C->mode == AtomMode::Dense;
@@ -1537,6 +1775,7 @@ private:
             d.lo0 = d.arity >= 1 ? C->layout.domain[pb][0] : 0;
             d.lo1 = d.arity >= 2 ? C->layout.domain[pb + 1][0] : 0;
             d.contiguous = pred_contiguous(p) ? 1 : 0;
+            d.magic = d.d1 >= 2 && d.size <= (u64{1} << 32) / d.d1 ? static_cast<u32>((u64{1} << 32) / d.d1 + 1) : 0;
             if (d.arity > 2 || !d.contiguous)
                 decode_arith = false;
             for (const DevPair& q : pairs)
@@ -1593,17 +1832,59 @@ private:
         h.num_goal_neg = static_cast<u32>(C->goal_neg.size());
         h.goal_unsat = C->goal_unsat ? 1 : 0;
         h.fluent_count = C->layout.fluent_count;
-        // hot sections first: everything read per state by the step and count kernels
+        // Steps and terms are records of 32 bytes at multiples of 32 bytes, and every reference to one is its index from the
+        // image's start; so are the word offsets of dom0 words and static rows in the terms. The kernels then reach all
+        // of a plan from the one image pointer.
+        static_assert(sizeof(DevStep) == 32 && sizeof(DevTerm) == 32);
+        auto align4 = [&] {
+            while (img.size() % 4)
+                img.push_back(0);
+        };
+        const u64 off_dom0 = put(dom0_words.data(), dom0_words.size() * sizeof(u64));
+        const u64 off_term_rows = put(term_rows.data(), term_rows.size() * sizeof(u64));
+        if (img.size() > 0xFFFFFFF0ull)
+            throw Error("the static relations' rows exceed the device image's 32-bit word offsets");
+        align4();
+        const u32 term0 = static_cast<u32>(img.size() / 4);
+        for (size_t k = 0; k < terms.size(); ++k)
+            if (terms[k].path == static_cast<u32>(TermPath::Image))
+                terms[k].base += static_cast<u32>(static_term[k] ? off_term_rows : off_dom0);
+        put(terms.data(), terms.size() * sizeof(DevTerm));
+        const u32 step0 = static_cast<u32>(img.size() / 4);
+        for (DevStep& st : steps)
+        {
+            st.term_begin += term0;
+            st.cons_end += term0;
+        }
+        put(steps.data(), steps.size() * sizeof(DevStep));
+        for (DevSchema& ds : schemas)
+        {
+            for (u32& v : ds.plan_begin)
+                v += step0;
+            for (u32& v : ds.filter_step)
+                v += step0;
+        }
+        for (DevWitness& wd : witness)
+            for (u32 k = 0; k < kMaxParams; ++k)
+            {
+                wd.filter[k] += step0;
+                wd.plan_lo[k] += step0;
+                wd.plan_hi[k] += step0;
+            }
+        for (DevDelta& d : deltas)
+        {
+            d.test_begin += step0;
+            d.plan_begin += step0;
+            d.plan_end += step0;
+        }
         h.off_schemas = put(schemas.data(), schemas.size() * sizeof(DevSchema));
-        h.off_steps = put(steps.data(), steps.size() * sizeof(DevStep));
-        h.off_cons = put(cons.data(), cons.size() * sizeof(DevCons));
+        h.off_deltas = put(deltas.data(), deltas.size() * sizeof(DevDelta));
         h.off_checks = put(checks.data(), checks.size() * sizeof(DevCheck));
         h.off_effects = put(effects.data(), effects.size() * sizeof(DevEffect));
         h.off_pairs = put(pairs.data(), pairs.size() * sizeof(DevPair));
         h.num_decode = static_cast<u32>(decode.size());
         h.decode_arith = decode_arith ? 1 : 0;
         h.off_decode = put(decode.data(), decode.size() * sizeof(DevPredDecode));
-        h.off_dom0 = put(dom0_words.data(), dom0_words.size() * sizeof(u64));
         {
             // lazy slots: room for every fluent goal literal (the lists grow as their atoms intern)
             std::vector<u32> gp = C->goal_pos, gn = C->goal_neg;
@@ -1632,9 +1913,6 @@ private:
                 offs[p] = C->layout.offset[p] == kNone64 ? 0 : C->layout.offset[p];
             h.off_pred_offset = put(offs.data(), offs.size() * sizeof(u64));
         }
-        h.hot_words = img.size();
-        for (const DevStep& st : steps)
-            h.max_step_words = std::max(h.max_step_words, st.words);
         // rs tables: per position n entries (u64)
         h.num_positions = static_cast<u32>(C->layout.rs.size());
         h.off_rs = reserve_words(static_cast<size_t>(h.num_positions) * n);
@@ -1647,13 +1925,6 @@ private:
             h.off_slot_of = put(so.data(), so.size() * sizeof(u32));
         }
         h.off_records = put(records.data(), records.size() * sizeof(u64));
-        {
-            // static row tables back to back (n * ow words each); DevCons.table holds the table index, the kernel
-            // multiplies by n * ow
-            h.off_static_rows = img.size();
-            for (const auto& t : m_row_data)
-                img.insert(img.end(), t.begin(), t.end());
-        }
         h.off_static_keys = put(static_key_words.data(), static_key_words.size() * sizeof(u64));
         for (auto& meta : static_meta)
             meta.keys += h.off_static_keys;
@@ -1666,6 +1937,7 @@ private:
         }
         h.off_witness = any_witness ? put(witness.data(), witness.size() * sizeof(DevWitness)) : 0;
         h.lazy = lazy ? 1 : 0;
+        h.simple = checks.empty() && C->label_width <= kLaneDepth + 1 ? 1 : 0;
         std::memcpy(img.data(), &h, sizeof(h));
         C->image = std::move(img);
     }
@@ -2130,8 +2402,9 @@ std::vector<std::pair<u64, u64>> intern_atoms(CompiledTask& C, const std::vector
     h.num_goal_neg = static_cast<u32>(C.goal_neg.size());
     h.goal_unsat = C.goal_unsat ? 1 : 0;
     std::memcpy(C.image.data(), &h, sizeof(h));
-    // the header and the goal lists (hot section), the slot table's changed words, the new records
-    ranges.emplace_back(0, h.hot_words);
+    // the header, the goal lists, the slot table's changed words, the new records
+    ranges.emplace_back(0, (sizeof(DevTaskHeader) + 7) / 8);
+    ranges.emplace_back(h.off_goal_pos, h.off_pred_arity);
     ranges.emplace_back(h.off_slot_of + lo / 2, h.off_slot_of + hi / 2 + 1);
     ranges.emplace_back(h.off_records + first, h.off_records + C.fluent_slots);
     return ranges;

@@ -185,6 +185,48 @@ struct DevCons
     u32 pad;
 };
 
+/// How the kernels read a constraint's candidate words (DevTerm::path).
+enum class TermPath : u32
+{
+    Image = 0,  // words of the image: the dom0 bits, rows of a static relation cut to the step's window
+    Words = 1,  // words of the wave's region (view, then state row) that fall on the window's words
+    Bits = 2,   // rows of the wave's region at any bit position
+};
+
+/// A DevCons resolved against its view pair and its step's window (same index), so that a wave reads one record per
+/// constraint: row r of the source (row0, or the bound object of parameter src minus row0; r >= rows reads as empty,
+/// rows = kNone: always inside) at base + r * stride. Image, Words: base and stride in words; Bits: in bits, the row
+/// being `stride` bits long and the window starting at its bit `delta`.
+struct DevTerm
+{
+    u32 path;
+    u32 neg;
+    u32 src;
+    u32 row0;
+    u32 rows;
+    u32 base;
+    u32 stride;
+    i32 delta;
+};
+
+/// One way an action changes a schema's successor count: its effect `effect` (position in the action's effect list),
+/// if the atom's bit changes, makes or unmakes the bindings whose literal is that atom. The literal's parameters are
+/// bound to the atom's objects (param[k] = term[k]: an action parameter, or -(object + 1)), the pairs eq must agree,
+/// with `tests` the steps from test_begin check the bound parameters, and steps [plan_begin, plan_end) count the rest.
+constexpr u32 kMaxDeltaTerms = 4;
+struct DevDelta
+{
+    u32 schema;
+    u32 effect;
+    u32 nbound;
+    u32 tests;
+    u32 test_begin;
+    u32 plan_begin, plan_end;
+    u32 neq;
+    i32 param[kMaxDeltaTerms], term[kMaxDeltaTerms];
+    i32 eq[2 * kMaxDeltaTerms];
+};
+
 struct DevCheck
 {
     u32 kind;  // CheckKind
@@ -202,10 +244,11 @@ struct DevStep
     u32 words;   // window words
     u32 cons_begin, cons_end;    // into the schema's DevCons
     u32 check_begin, check_end;  // into the schema's DevCheck
-    u32 pad;
+    u32 term_begin;  // the terms to AND: [term_begin, cons_end) (the leading dom0 left out where another term implies it)
 };
 
 constexpr u32 kMaxParams = 32;
+constexpr u32 kLaneDepth = 3;  // levels of a lane's nested count that the kernels unroll
 
 /// Per schema: plans P_j (j = 0..arity) count the bindings with parameters [0, j) bound; filters F_i (i < arity) give
 /// the candidates of parameter i with [0, i) bound (the lexicographic pick).
@@ -218,7 +261,8 @@ struct DevSchema
     u32 filter_step[kMaxParams];     // the DevStep of filter i
     u32 eff_begin, eff_end;          // into effects
     u32 nadd;                        // effects [eff_begin, eff_begin + nadd) add, the rest delete
-    u32 affects;  // bit s: an action of this schema can change schema s's successor count (every bit past 32 schemas)
+    u32 recount;  // bit s: schema s is counted again after an action of this schema (every bit past 32 schemas)
+    u32 del_begin, add_begin, add_end;  // DevDelta: counts taken away before the move, then counts added after it
 };
 
 /// Witness pruning of a schema (the parameters no effect mentions, witnesses, bound last and only once per binding of
@@ -243,6 +287,7 @@ struct DevEffect
     u64 base;
     u32 var_param[4];
     u32 var_pos[4];  // global position index into the rs tables
+    i32 terms[2];    // the first two terms: a parameter, or -(object + 1)
 };
 
 /// A view pair: the rows of a fluent predicate of arity 1 (one row) or 2 (forward: source position 0, or backward).
@@ -271,7 +316,7 @@ struct DevPredDecode
     u32 lo0, lo1;
     u32 contiguous;  // every position's domain is a contiguous object range
     u32 has_scatter; // some view pair of the predicate is built by scattering set bits
-    u32 pad;
+    u32 magic;       // x / d1 = the high word of x * magic for x < size (0: divide)
 };
 
 struct DevTaskHeader
@@ -289,22 +334,21 @@ struct DevTaskHeader
     u32 goal_unsat;
     u64 fluent_count;
     // word offsets into the image
-    u64 off_schemas, off_steps, off_cons, off_checks, off_effects, off_pairs;
-    u64 off_rs, off_slot_of, off_records, off_dom0, off_static_rows, off_static_keys, off_static_meta;
+    u64 off_schemas, off_checks, off_effects, off_pairs;
+    u64 off_rs, off_slot_of, off_records, off_static_keys, off_static_meta;
     u64 off_goal_pos, off_goal_neg, off_initial;
     u64 off_pred_arity, off_pos_begin;
     u64 off_pred_pairs;   // per predicate: view pair of the unary / forward rows (low 32 bits), backward (high)
     u64 off_pred_offset;  // per predicate: first canonical id (u64)
     u64 off_decode;       // DevPredDecode per fluent predicate with atoms, ascending offset
-    u64 hot_words;        // the image's first hot_words words hold everything the kernels read per state
-                          // (staged in LDS); rs tables, slot tables, records, static rows and keys follow
     u32 num_positions;
     u32 num_decode;
     u32 decode_arith;     // 1: slots decode arithmetically (dense slots, contiguous domains)
     u32 init_count;     // successors of the initial state (filled once the device has counted them)
-    u32 max_step_words; // the widest candidate window of any plan or filter step, in words
     u32 lazy;           // 1: lazy slots (slot_of, records, goal lists and initial row sized for every canonical atom)
+    u32 simple;         // no checks, and every schema has at most kLaneDepth + 1 parameters
     u32 pad;
+    u64 off_deltas;     // DevDelta
     u64 off_witness;    // DevWitness per schema (0: no schema has a witness parameter)
 };
 

@@ -15,8 +15,35 @@ def test_search_fingerprint_over_row_widths(props, atoms):
     from mymyr_amd.task import Task
     from oracle import port
 
-    text = gen.random_strips(props, 60, init_atoms=max(3, props // 8), goal_atoms=2, seed=4)
+    text = gen.random_strips(props, 4 * props, init_atoms=max(3, props // 8), goal_atoms=2, seed=4)
     kw = dict(max_depth=2, stop_at_goal=False)
     r = search.brfs(Task.from_text(text, atoms), fingerprint=True, **kw)
     p = port.brfs(port.Task(text, "dense"), max_states=1 << 40, **kw)
     assert (r.states, r.fingerprint) == (p["states"], p["fingerprint"])
+
+
+TASKS = ["blocks__probBLOCKS-8-0", "gripper__prob05", "logistics00__probLOGISTICS-6-1", "miconic__s7-4", "zenotravel__p05",
+         "driverlog__p03", "depot__p02", "rovers__p02", "freecell__p02", "pegsol-08-strips__p22", "sokoban-opt08-strips__p14",
+         "visitall__visitall_x-6_y-3_r-100", "snake-opt18-strips__p05", "parcprinter-opt11-strips__p03", "pathways__p02",
+         "transport-opt08-strips__p23", "noop_switches", "witness_order_0", "gridworld", "transport", "strips"]
+
+
+@pytest.mark.parametrize("name", TASKS)
+def test_counts_after_a_move_equal_a_recount(name, golden):
+    """A step brings the successor counts up to date from the move's changed atoms (and the cache row's fingerprint from
+    its changed words), and a refresh counts the same states from nothing: the same counts and cache rows, over domains
+    whose literals share predicates, repeat objects, are negative, ground or of three and more terms."""
+    import torch
+
+    from mymyr_amd import rl
+    from mymyr_amd.task import Task
+
+    pool = rl.DeviceEnvPool(Task.from_text_file(golden.task_path(name)), 96, seed=11, max_steps=25)
+    pool.reset()
+    for k in range(40):
+        pool.step()
+        count, cache = pool.count.clone(), pool.counts_cache.clone()
+        pool.refresh()
+        assert torch.equal(count, pool.count), f"{name}: counts at step {k}"
+        assert torch.equal(cache, pool.counts_cache), f"{name}: cache rows at step {k}"
+    pool.check()
