@@ -291,6 +291,7 @@ void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const in
         out->total = dropping ? totals[1] : generated;
         if (out->offsets)
             launch_offsets_i32(offs, rows + 1, out->offsets, stream);
+        const bool hash_rows = out->succ_hash && out->succ && out->words >= T.W && !lazy;
         const bool rows_out = out->succ || out->parent || out->schema || out->binding || out->goal || out->succ_hash || out->noop ||
                               out->index;
         if ((rows_out && out->capacity) || (out->succ && out->words < T.W))
@@ -304,11 +305,15 @@ void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const in
             a.schema = out->schema;
             a.binding = out->binding;
             a.goal = out->goal;
-            a.succ_hash = out->succ_hash;
+            // whole rows are hashed where they were written, 64 rows side by side (one row's hash is a serial chain); rows
+            // narrower than the task's in the expansion, which sees the words that do not fit
+            a.succ_hash = hash_rows ? nullptr : out->succ_hash;
             a.noop = out->noop;
             a.index = out->index;
             launch_expand(a, stream);
         }
+        if (hash_rows)
+            launch_hash_rows(out->succ, std::min<u64>(out->total, out->capacity), out->words, out->succ_hash, stream);
         hip_check(hipMemcpyAsync(st, words_status, sizeof(st), hipMemcpyDeviceToHost, stream), "expand status");
         hip_check(hipStreamSynchronize(stream), "expand");
         // lazy slots: successors that added atoms without a slot are written again once those atoms are interned

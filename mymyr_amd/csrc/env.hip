@@ -323,6 +323,42 @@ __global__ void k_kept_counts(const u32* counts, const u32* noops, u64 rows, u32
 // Padded view of a flat expansion, one wave per row: the row's k slots are contiguous in every output, so the lanes
 // walk each output row (scalars over the k slots, succ over k * words, binding over k * label_width) with coalesced
 // stores, reading the flat rows b .. b + k - 1 that are also contiguous.
+template<class X>
+__device__ __forceinline__ void pad_rows(X* dst, const X* src, u32 K, u32 n, u32 W, u32 FW, X fill, u32 lane)
+{
+    if (W == 0)
+        return;
+    const u32 dk = kWave / W, dw = kWave % W;
+    u32 k = lane / W, w = lane % W;
+    constexpr int kBatch = 4;  // loads of a lane in flight before their stores
+    while (k < K)
+    {
+        X v[kBatch];
+        u64 at[kBatch];
+        bool live[kBatch];
+#pragma unroll
+        for (int q = 0; q < kBatch; ++q)
+        {
+            live[q] = k < K;
+            at[q] = static_cast<u64>(k) * W + w;
+            v[q] = fill;
+            if (k < n && w < FW)
+                v[q] = src[static_cast<u64>(k) * FW + w];
+            k += dk;
+            w += dw;
+            if (w >= W)
+            {
+                w -= W;
+                ++k;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kBatch; ++q)
+            if (live[q])
+                dst[at[q]] = v[q];
+    }
+}
+
 __global__ __launch_bounds__(256) void k_pad(PadArgs a)
 {
     const u32 lane = lane_id();
@@ -364,25 +400,19 @@ __global__ __launch_bounds__(256) void k_pad(PadArgs a)
         }
         if (a.out_succ)
         {
+            // rows of equal even widths go 16 bytes a lane; the lanes' (slot, word) advance by a wave's stride without a
+            // division per element
             const u32 W = a.words, FW = a.succ ? a.flat_words : 0;
-            u64* dst = a.out_succ + base * W;
-            const u64 total = u64{K} * W;
-            for (u64 t = lane; t < total; t += kWave)
-            {
-                const u32 k = static_cast<u32>(t / W), w = static_cast<u32>(t - u64{k} * W);
-                dst[t] = k < n && w < FW ? a.succ[(b + k) * FW + w] : 0;
-            }
+            if (W == FW && (W & 1) == 0 && ((reinterpret_cast<std::uintptr_t>(a.out_succ) | reinterpret_cast<std::uintptr_t>(a.succ)) & 15) == 0)
+                pad_rows<ulonglong2>(reinterpret_cast<ulonglong2*>(a.out_succ) + base * (W / 2), reinterpret_cast<const ulonglong2*>(a.succ) + b * (FW / 2),
+                                     K, n, W / 2, FW / 2, ulonglong2{0, 0}, lane);
+            else
+                pad_rows<u64>(a.out_succ + base * W, a.succ + b * FW, K, n, W, FW, u64{0}, lane);
         }
         if (a.out_binding)
         {
             const u32 L = a.label_width, FL = a.binding ? a.flat_label_width : 0;
-            i32* dst = a.out_binding + base * L;
-            const u64 total = u64{K} * L;
-            for (u64 t = lane; t < total; t += kWave)
-            {
-                const u32 k = static_cast<u32>(t / L), w = static_cast<u32>(t - u64{k} * L);
-                dst[t] = k < n && w < FL ? a.binding[(b + k) * FL + w] : -1;
-            }
+            pad_rows<i32>(a.out_binding + base * L, a.binding + b * FL, K, n, L, FL, -1, lane);
         }
     }
 }

@@ -898,11 +898,14 @@ __device__ __forceinline__ u32 for_each_successor(const TaskDev& T, const Tab& H
 /// The slot of an effect's atom under the wave's binding (kNone: none); its canonical id in *cid.
 __device__ __forceinline__ u32 effect_slot(const TaskDev& T, const Lds& L, const DevEffect& e, u64* cid_out)
 {
-    u64 cid = e.base;
+    u64 cid = e.arith ? e.arith_base : e.base;
 #pragma unroll
     for (u32 v = 0; v < 4; ++v)
         if (v < e.nvar)
-            cid += T.rs[static_cast<u64>(e.var_pos[v]) * T.n + L.ub[e.var_param[v]]];
+        {
+            const u32 o = L.ub[e.var_param[v]];
+            cid += e.arith ? o * e.mul[v] : T.rs[static_cast<u64>(e.var_pos[v]) * T.n + o];
+        }
     *cid_out = cid;
     if (cid >= T.fluent_count)
         return kNone;
@@ -1819,7 +1822,7 @@ __device__ __forceinline__ void expand_row(const ExpandArgs& A, const TaskDev& T
         {
             const u64 pos = A.offsets[i] - A.offset_base + (A.drop_noops ? kept : k);
             ++kept;
-            const u32 n = (A.succ || A.succ_hash) ? trimmed_words(L.row, T.W, lane) : 0;
+            const u32 n = (A.succ_hash || (A.succ && A.out_words < T.W)) ? trimmed_words(L.row, T.W, lane) : 0;
             const bool fits = n <= A.out_words;
             if (A.succ && !fits && lane == 0)
                 atomicMax(A.words_needed, n);

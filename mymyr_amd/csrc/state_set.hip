@@ -50,6 +50,65 @@ __global__ __launch_bounds__(kBlock) void k_hash_rows(const u64* __restrict__ ro
         out[j] = h;
 }
 
+/// hash_state of rows wider than a lane group's registers hold cheaply, a lane per row. The hash is a chain of one
+/// multiply-fold per word pair, so a group that shares a row computes it in every lane; here 64 rows' chains run side by
+/// side, and the wave reads the rows 16 words at a time through LDS (whole 128-byte lines, rows padded to 17 words so
+/// that the lanes' reads of one word fall on different banks). The chain starts from the trimmed length, found from the
+/// rows' last tiles first. Bound by the multiplies and the reads: 10^6 rows of 176 words, see launch_hash_rows.
+constexpr u32 kHashTile = 16;
+constexpr int kHashWaves = 4;
+__global__ __launch_bounds__(kHashWaves * kWave) void k_hash_long(const u64* __restrict__ rows, u64 n, u32 words, u64* __restrict__ out)
+{
+    __shared__ u64 tiles[kHashWaves][kWave * (kHashTile + 1)];
+    const u32 lane = lane_id(), wave = threadIdx.x / kWave;
+    u64* tile = tiles[wave];
+    const u64* mine = tile + lane * (kHashTile + 1);
+    const u64 first = (static_cast<u64>(blockIdx.x) * kHashWaves + wave) * kWave;
+    if (first >= n)
+        return;  // whole waves: barriers below are wave-wide
+    const u32 count = static_cast<u32>(min(static_cast<u64>(kWave), n - first));
+    const u32 last = (words - 1) / kHashTile;
+    // words [16 t, 16 t + 16) of the wave's rows (zeros past the rows' words): lanes 16 r + c take word c of row 4 k + r
+    auto load = [&](u32 t) {
+        const u32 c = lane % kHashTile, w = t * kHashTile + c;
+        u64 v[kHashTile];
+#pragma unroll
+        for (u32 k = 0; k < kHashTile; ++k)
+        {
+            const u32 r = k * (kWave / kHashTile) + lane / kHashTile;
+            v[k] = r < count && w < words ? rows[(first + r) * words + w] : 0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (u32 k = 0; k < kHashTile; ++k)
+            tile[(k * (kWave / kHashTile) + lane / kHashTile) * (kHashTile + 1) + c] = v[k];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    u32 len = 0;  // 1 + the highest nonzero word
+    for (u32 t = last + 1; t > 0 && __ballot(len == 0 && lane < count); --t)
+    {
+        load(t - 1);
+        for (u32 c = 0; c < kHashTile; ++c)
+            if (mine[c] && len < (t - 1) * kHashTile + c + 1 && (len == 0 || len > (t - 1) * kHashTile))
+                len = (t - 1) * kHashTile + c + 1;
+    }
+    u64 h = kHashSeed ^ (static_cast<u64>(len) * kHashP1);
+    for (u32 t = 0; __ballot(t * kHashTile < len); ++t)
+    {
+        load(t);
+#pragma unroll
+        for (u32 c = 0; c < kHashTile; c += 2)
+            if (t * kHashTile + c < len)
+                h = mulfold(h ^ mine[c] ^ kHashP1, mine[c + 1] ^ kHashP2);
+    }
+    if (lane < count)
+        out[first + lane] = mix64(h);
+}
+
 template<int G, int K>
 __global__ __launch_bounds__(kBlock) void k_insert(StateSetView s, const u64* __restrict__ rows, u64 n, u64* __restrict__ cand_slot,
                                                   u8* __restrict__ flags, u32* __restrict__ status, BlockedView blocked)
@@ -298,13 +357,19 @@ void launch_dedup_rows(u64 start, u64 count, u32 words, u64 seed, double dup, u6
     launch_check("dedup rows");
 }
 
+/// Rows up to this many words are hashed by a lane group each, wider ones by a lane each.
+constexpr u32 kGroupHashWords = 16;
+
 void launch_hash_rows(const u64* rows, u64 n, u32 words, u64* out, hipStream_t stream)
 {
     if (n == 0)
         return;
-    with_shape(words, [&]<int G, int K>() {
-        hipLaunchKernelGGL((k_hash_rows<G, K>), dim3(group_blocks<G>(n)), dim3(kBlock), 0, stream, rows, n, words, out);
-    });
+    if (words > kGroupHashWords)
+        hipLaunchKernelGGL(k_hash_long, dim3(blocks_for(n, kHashWaves * kWave)), dim3(kHashWaves * kWave), 0, stream, rows, n, words, out);
+    else
+        with_shape(words, [&]<int G, int K>() {
+            hipLaunchKernelGGL((k_hash_rows<G, K>), dim3(group_blocks<G>(n)), dim3(kBlock), 0, stream, rows, n, words, out);
+        });
     launch_check("hash_rows");
 }
 

@@ -1442,6 +1442,25 @@ private:
                             ++e.nvar;
                         }
                     }
+                    e.arith = 1;
+                    e.arith_base = e.base;
+                    for (u32 v = 0; v < e.nvar; ++v)
+                    {
+                        const std::vector<u32>& dom = C->layout.domain[e.var_pos[v]];
+                        const std::vector<u64>& rs = C->layout.rs[e.var_pos[v]];
+                        bool line = !dom.empty();
+                        for (size_t r = 1; r < dom.size(); ++r)
+                            line = line && dom[r] == dom[0] + r;
+                        for (u32 o = 0; o < n && line; ++o)
+                            line = !test_bit(C->dom0[si][e.var_param[v]], o) || (o >= dom[0] && o - dom[0] < dom.size());
+                        if (!line)
+                        {
+                            e.arith = 0;
+                            break;
+                        }
+                        e.mul[v] = dom.size() > 1 ? rs[dom[1]] - rs[dom[0]] : 0;
+                        e.arith_base += rs[dom[0]] - dom[0] * e.mul[v];
+                    }
                     effects.push_back(e);
                 }
             ds.eff_end = static_cast<u32>(effects.size());

@@ -288,6 +288,10 @@ struct DevEffect
     u32 var_param[4];
     u32 var_pos[4];  // global position index into the rs tables
     i32 terms[2];    // the first two terms: a parameter, or -(object + 1)
+    u32 arith;       // 1: cid = arith_base + sum of object * mul (every variable position's domain is a contiguous range
+    u32 pad;         // that holds the parameter's static domain), so no table is read
+    u64 arith_base;
+    u64 mul[4];
 };
 
 /// A view pair: the rows of a fluent predicate of arity 1 (one row) or 2 (forward: source position 0, or backward).

@@ -744,7 +744,7 @@ def expand(task: Task | TaskTable, states: torch.Tensor, *, task_ids: torch.Tens
         capacity = probe.generated
     dev = s.device
     cap = int(capacity)
-    succ = torch.zeros((cap, ow), dtype=torch.int64, device=dev)
+    succ = torch.empty((cap, ow), dtype=torch.int64, device=dev)  # every kept row is written whole
     parent = torch.empty(cap, dtype=torch.int32, device=dev)
     schema = torch.empty(cap, dtype=torch.int32, device=dev)
     binding = torch.empty((cap, L), dtype=torch.int32, device=dev)

@@ -47,3 +47,54 @@ def test_counts_after_a_move_equal_a_recount(name, golden):
         assert torch.equal(count, pool.count), f"{name}: counts at step {k}"
         assert torch.equal(cache, pool.counts_cache), f"{name}: cache rows at step {k}"
     pool.check()
+
+
+@pytest.mark.parametrize("words", [16, 17, 18, 31, 32, 33, 47, 176, 200, 1025])
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 257])
+def test_hash_of_wide_rows(words, rows):
+    """Rows hashed by a lane each, 64 to a wave and 16 words at a time: row counts around a wave, widths around a tile,
+    rows whose trimmed length ends anywhere (an empty row included)."""
+    import torch
+
+    from mymyr_amd import hip
+    from oracle import port
+
+    rng = np.random.default_rng(words * 1000 + rows)
+    a = rng.integers(0, 1 << 63, size=(rows, words), dtype=np.uint64)
+    for i in range(rows):
+        a[i, rng.integers(0, words + 1):] = 0
+    a[rows // 2] = 0
+    got = hip.hash_rows(torch.from_numpy(a.view(np.int64)).cuda()).cpu().numpy().view(np.uint64)
+    assert [int(x) for x in got] == [port.hash_state(r) for r in a]
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("k", [1, 7, 40])
+def test_pad_of_rows_at_any_alignment(k, shift):
+    """The padded view of rows of an even width (16 bytes a lane), and of the same rows starting 8 bytes off."""
+    import torch
+
+    from mymyr_amd import gen, rl
+    from mymyr_amd.task import Task
+    from oracle import port
+
+    t = Task.from_text(gen.transport(24, 6, 42, goals=6, seed=2))
+    assert t.words % 2 == 0
+    pool = rl.DeviceEnvPool(t, 33, seed=3)
+    pool.reset()
+    pool.step()
+    x = rl.expand(t, pool.states, goal=True, hashes=True)
+    n = x["succ"].shape[0]
+    buf = torch.empty(n * t.words + shift, dtype=torch.int64, device="cuda")
+    buf[shift:] = x["succ"].reshape(-1)
+    flat = dict(x, succ=buf[shift:].view(n, t.words))
+    p = rl.pad(flat, k)
+    off = x["offsets"].cpu().numpy()
+    succ, bind = x["succ"].cpu().numpy(), x["binding"].cpu().numpy()
+    for i in range(33):
+        c = min(k, int(off[i + 1] - off[i]))
+        row = p["succ"][i].cpu().numpy()
+        assert np.array_equal(row[:c], succ[off[i]: off[i] + c]) and not row[c:].any()
+        b = p["binding"][i].cpu().numpy()
+        assert np.array_equal(b[:c], bind[off[i]: off[i] + c]) and (b[c:] == -1).all()
+    assert [int(h) for h in x["succ_hash"].cpu().numpy().view(np.uint64)] == [port.hash_state(r) for r in succ.view(np.uint64)]
