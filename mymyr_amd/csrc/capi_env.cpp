@@ -249,6 +249,9 @@ void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const in
             a.instances = env->instances();
             a.wave_words = env->wave_words;
             a.general = env->general;
+            a.table_words = env->words;
+            for (const TaskDev* t : inst)
+                a.unlistable |= t->listable ? 0u : 1u;
         }
         a.states = states;
         a.rows = rows;

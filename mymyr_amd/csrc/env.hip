@@ -55,6 +55,7 @@ TaskDev task_dev(const u64* img, const DevTaskHeader& h)
     t.lazy = h.lazy;
     t.missing = nullptr;
     t.simple = h.simple;
+    t.listable = h.listable;
     set_region(t);
     return t;
 }
@@ -589,11 +590,15 @@ void launch_expand(const ExpandArgs& args, hipStream_t stream)
         return;
     ExpandArgs a = args;
     a.wave_words = wave_words_of(a.wave_words, a.T);
+    const bool simple = a.T.simple && !a.general;
+    // successors 64 at a time, where every instance is listable and the call asks for whole rows (rows narrower than the
+    // task's need their trimmed lengths, a successor at a time)
+    a.list = simple && a.T.listable && !a.unlistable && !a.witness && !a.succ_hash && (!a.succ || (!a.tasks && a.out_words >= a.T.W) || (a.tasks && a.out_words >= a.table_words));
     size_t lds = 0;
-    const unsigned nw = block_shape(static_cast<size_t>(a.wave_words) * 8, &lds);
+    const unsigned nw = block_shape(static_cast<size_t>(a.wave_words + (a.list ? kListCap : 0)) * 8, &lds);
     if (a.witness && a.tasks)
         throw std::invalid_argument("mymyr_amd: expand: witness pruning over a task table is not supported by the device expansion");
-    const EnvKernels k = kernels_for(a.T.simple && !a.general);
+    const EnvKernels k = kernels_for(simple);
     const auto fn = a.tasks ? k.expand_table : a.witness ? k.expand_witness : k.expand;
     set_lds(reinterpret_cast<const void*>(fn), lds);
     hipLaunchKernelGGL(fn, dim3(grid_for(a.rows, nw)), dim3(nw * kWave), lds, stream, a);

@@ -217,6 +217,9 @@ struct ExpandArgs
     u32 instances;
     u32 wave_words;        // LDS words per wave (0: T's)
     u32 general;           // some instance is not simple (one instance: T tells)
+    u32 unlistable;        // some instance is not listable (one instance: T tells)
+    u32 table_words;       // over a table: the widest instance's words
+    u32 list;              // set by launch_expand: successors are listed 64 at a time
     const u64* states;
     u64 rows;
     u32 words;

@@ -1780,10 +1780,215 @@ __device__ __forceinline__ u32 witness_counts(const TaskDev& T, const Tab& H, co
     return total;
 }
 
+/// A lane's bindings of schema parameters [I, arity) that complete its binding, in lexicographic order: packed (16 bits
+/// per object) into list[index - lo] for the indices in [lo, hi), the first of them `index`.
+template<u32 I>
+__device__ __forceinline__ void list_lanes(const Tab& H, const Lds& L, const auto& S, u32 arity, u64 prefix, u32& index, u32 lo, u32 hi,
+                                           lds<u64>* list, u32 lane)
+{
+    const DevStep F = ld(H.steps + S.filter_step[I]);
+    for (u32 w = 0; w < F.words; ++w)
+        for (u64 m = cand_word(H, L, F, w, lane); m; m &= m - 1)
+        {
+            const u32 o = F.lo + 64 * w + static_cast<u32>(__builtin_ctzll(m));
+            const u64 e = prefix | (static_cast<u64>(o) << (16 * I));
+            if (I + 1 == arity)
+            {
+                if (index >= lo && index < hi)
+                    list[index - lo] = e;
+                ++index;
+            }
+            else if constexpr (I < kLaneDepth)
+            {
+                L.bind[I * 64 + lane] = o;
+                list_lanes<I + 1>(H, L, S, arity, e, index, lo, hi, list, lane);
+            }
+        }
+}
+
+/// The successors of the state in canonical order, kListCap at a time, for listable tasks (TaskDev::listable). Each schema's
+/// first parameter's candidates are spread over the lanes, which count their completions (their places in the list) and
+/// then write their bindings there; the list is handed on 64 successors at a time: flush(s, first, n) with the bindings
+/// of successors [0, n) at list[first ..].
+template<class Flush>
+__device__ __forceinline__ void for_each_listed(const TaskDev& T, const Tab& H, const Lds& L, lds<u64>* list, u32 lane, Flush&& flush)
+{
+    for (u32 s = 0; s < T.num_schemas; ++s)
+    {
+        if (uni(L.counts[s]) == 0)
+            continue;
+        const auto& S = H.schemas[s];
+        const u32 arity = S.arity;
+        if (arity == 0)
+        {
+            if (lane == 0)
+                list[0] = 0;
+            wave_sync();
+            flush(s, 0u, 1u);
+            continue;
+        }
+        const DevStep F = ld(H.steps + S.filter_step[0]);
+        const u32 pb = S.plan_begin[1], pe = S.plan_begin[2];
+        for_nonzero_words(T, H, L, F, 0, lane, [&](u32 w, u64 m) {
+            const u32 o = F.lo + 64 * w + lane;
+            u32 c = 0;
+            if ((m >> lane) & 1)
+            {
+                L.bind[lane] = o;
+                c = count_lanes<kLaneDepth>(T, H, L, pb, pe, lane);
+            }
+            const u32 incl = wave_inclusive(c), total = lane_value(incl, kWave - 1), at = incl - c;
+            for (u32 lo = 0; lo < total; lo += kListCap)
+            {
+                const u32 hi = min(total, lo + kListCap);
+                wave_sync();
+                if (c && at < hi && incl > lo)
+                {
+                    if (arity == 1)
+                        list[at - lo] = o;
+                    else
+                    {
+                        u32 index = at;
+                        list_lanes<1>(H, L, S, arity, o, index, lo, hi, list, lane);
+                    }
+                }
+                wave_sync();
+                for (u32 b = lo; b < hi; b += kWave)
+                    flush(s, b - lo, min(static_cast<u32>(kWave), hi - b));
+            }
+            return false;
+        });
+    }
+}
+
+/// The expansion of a row of a listable task (as expand_row), 64 successors at a time: each lane forms one successor's
+/// effect slots, flags and label from its binding, then the wave writes the successor rows one after the other, the
+/// parent's words with the effects' bits patched in registers.
+__device__ __forceinline__ void expand_listed(const ExpandArgs& A, const TaskDev& T, const Tab& H, const Lds& L, lds<u64>* list, u64 i, u32 c,
+                                              u32 lane)
+{
+    const bool drop = A.drop_noops != 0;
+    const bool write = A.pass == 1;
+    const bool keep_all = write && drop && uni(A.noops[i]) == c;
+    const u64 out0 = write ? A.offsets[i] - A.offset_base : 0;
+    u32 listed = 0, kept = 0, noops = 0;
+    for_each_listed(T, H, L, list, lane, [&](u32 s, u32 first, u32 n) {
+        const auto& S = H.schemas[s];
+        const u32 eff = S.eff_begin, ne = S.eff_end - eff, nadd = S.nadd;
+        const bool mine = lane < n;
+        const u64 bind = mine ? list[first + lane] : 0;
+        // the lane's successor: its effects' slots, and whether it changes a bit (delete, then add)
+        u32 sl[kListEff];
+        bool changed = false;
+#pragma unroll
+        for (u32 j = 0; j < kListEff; ++j)
+        {
+            sl[j] = kNone;
+            if (j >= ne)
+                continue;
+            const DevEffect e = ld(H.effects + eff + j);
+            u64 cid = e.arith ? e.arith_base : e.base;
+#pragma unroll
+            for (u32 v = 0; v < 4; ++v)
+                if (v < e.nvar)
+                {
+                    const u32 o = static_cast<u32>(bind >> (16 * e.var_param[v])) & 0xFFFF;
+                    cid += e.arith ? o * e.mul[v] : T.rs[static_cast<u64>(e.var_pos[v]) * T.n + o];
+                }
+            if (mine && cid < T.fluent_count)
+                sl[j] = T.dense ? static_cast<u32>(cid) : T.slot_of[cid];
+            if (mine && j < nadd && sl[j] == kNone)
+                missing_atom(T, cid, A.status);
+        }
+        auto bit = [&](u32 q) {  // bit q of the lane's successor
+            bool v = q < 64 * T.W && row_bit(L.row, q);
+#pragma unroll
+            for (u32 j = kListEff; j-- > 0;)  // deletes (last) first, so that the adds win
+                if (j < ne && sl[j] == q)
+                    v = j < nadd;
+            return v;
+        };
+#pragma unroll
+        for (u32 j = 0; j < kListEff; ++j)
+            if (j < ne && sl[j] != kNone)
+                changed = changed || bit(sl[j]) != row_bit(L.row, sl[j]);
+        const bool noop = !changed;
+        noops += static_cast<u32>(__popcll(__ballot(mine && noop)));
+        const bool take = mine && (!drop || !noop || keep_all);
+        const u64 took = __ballot(take);
+        const u32 k = listed + lane;
+        const u64 pos = out0 + (drop ? kept + static_cast<u32>(__popcll(took & ((u64{1} << lane) - 1))) : k);
+        listed += n;
+        kept += static_cast<u32>(__popcll(took));
+        const bool out = write && take && pos < A.capacity;
+        if (out)
+        {
+            if (A.goal)
+            {
+                bool g;
+                if (A.any_goal.any)
+                    g = any_of_holds_dev(A.any_goal, bit);
+                else
+                {
+                    g = !T.goal_unsat;
+                    for (u32 q = 0; q < T.ngp; ++q)
+                        g = g && bit(H.goal_pos[q]);
+                    for (u32 q = 0; q < T.ngn; ++q)
+                        g = g && !bit(H.goal_neg[q]);
+                }
+                A.goal[pos] = g ? 1 : 0;
+            }
+            if (A.noop)
+                A.noop[pos] = noop ? 1 : 0;
+            if (A.index)
+                A.index[pos] = static_cast<i32>(k);
+            if (A.parent)
+                A.parent[pos] = static_cast<i32>(i);
+            if (A.schema)
+                A.schema[pos] = static_cast<i32>(s);
+            if (A.binding)
+                for (u32 q = 0; q < A.label_width; ++q)
+                    A.binding[pos * A.label_width + q] = q < S.arity ? static_cast<i32>((bind >> (16 * q)) & 0xFFFF) : -1;
+        }
+        if (!A.succ)
+            return;
+        for (u64 x = __ballot(out); x; x &= x - 1)
+        {
+            const u32 j = static_cast<u32>(__builtin_ctzll(x));
+            u64* const dst = A.succ + lane_value(pos, j) * A.out_words;
+            u32 es[kListEff];
+#pragma unroll
+            for (u32 q = 0; q < kListEff; ++q)
+                es[q] = q < ne ? lane_value(sl[q], j) : kNone;
+            for (u32 w = lane; w < A.out_words; w += kWave)
+            {
+                u64 v = w < T.W ? L.row[w] : 0;
+#pragma unroll
+                for (u32 q = kListEff; q-- > 0;)
+                    if (q < ne && w == es[q] >> 6 && es[q] != kNone)
+                    {
+                        const u64 b = u64{1} << (es[q] & 63);
+                        v = q < nadd ? v | b : v & ~b;
+                    }
+                dst[w] = v;
+            }
+        }
+    });
+    if (listed != c && lane == 0)
+        atomicOr(A.status, kStatusPickFailed);
+    if (A.pass == 0 && lane == 0)
+    {
+        A.counts[i] = c;
+        A.noops[i] = noops;
+    }
+    wave_sync();
+}
+
 /// The expansion of row i (pass 0: its counts and the validation of its words; pass 1: its successors from
 /// offsets[i] on) with the tables of its instance.
 template<bool kWitness>
-__device__ __forceinline__ void expand_row(const ExpandArgs& A, const TaskDev& T, const Tab& H, const Lds& L, u64 i, u32 lane)
+__device__ __forceinline__ void expand_row(const ExpandArgs& A, const TaskDev& T, const Tab& H, const Lds& L, [[maybe_unused]] lds<u64>* list, u64 i,
+                                           u32 lane)
 {
     const u32 Lw = A.label_width;
     const u64* src = A.states + i * A.words;
@@ -1813,6 +2018,12 @@ __device__ __forceinline__ void expand_row(const ExpandArgs& A, const TaskDev& T
             A.counts[i] = c;
         return;
     }
+    if constexpr (!kGeneral && !kWitness)
+        if (A.list)
+        {
+            expand_listed(A, T, H, L, list, i, c, lane);
+            return;
+        }
     const bool keep_all = A.pass == 1 && A.drop_noops && A.noops[i] == c;
     u32 noops = 0, kept = 0;
     const u32 listed = for_each_successor<kWitness>(T, H, L, lane, [&](u32 k, u32 s) {
@@ -1889,7 +2100,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void k_expand(ExpandArgs A)
 {
     extern __shared__ u64 smem[];
     const u32 lane = lane_id(), wave = uni(threadIdx.x / kWave), nw = blockDim.x / kWave;
-    lds<u64>* const region = (lds<u64>*)smem + static_cast<u64>(wave) * A.wave_words;
+    lds<u64>* const region = (lds<u64>*)smem + static_cast<u64>(wave) * (A.wave_words + (A.list ? kListCap : 0));
     for (u64 i = static_cast<u64>(blockIdx.x) * nw + wave; i < A.rows; i += static_cast<u64>(gridDim.x) * nw)
     {
         u32 k = 0;
@@ -1913,7 +2124,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void k_expand(ExpandArgs A)
         }
         const ExpandArgs& a = kernel_args<ExpandArgs>();
         const TaskDev& T = kOne ? a.T : instance_tables(a.tasks, k);
-        expand_row<kWitness>(a, T, tab_of(T), lds_of(region, T), i, lane);
+        expand_row<kWitness>(a, T, tab_of(T), lds_of(region, T), region + A.wave_words, i, lane);
     }
 }
 

@@ -37,6 +37,7 @@ struct TaskDev
     u32 n, ow, W, num_schemas, num_pairs, view_words, ngp, ngn, goal_unsat, dense, label_width, fluent_slots;
     u32 num_decode, decode_arith;
     u32 simple;    // no literal is checked one by one and no schema has more than kLaneDepth + 1 parameters
+    u32 listable;  // simple, at most kListEff effects per schema and objects of 16 bits: successors are listed (expand_listed)
     u32 lazy;      // lazy slots: an added atom without a slot is recorded in `missing`
     u64* missing;  // lazy slots: bit per canonical fluent atom (device; set by the successor kernels), else null
     u32 l_row, l_dfs_m, l_ub, l_bind, l_counts, l_dfs_w, l_eff, l_before, l_cur, l_words;  // a wave's LDS region (set_region)
@@ -47,6 +48,7 @@ struct TaskDev
 TaskDev task_dev(const u64* image_dev, const DevTaskHeader& h);
 
 constexpr u32 kMaxEnvSchemas = 8192;  // schemas whose per-state counts a wave keeps in LDS
+constexpr u32 kListCap = 128;      // successors listed at a time (a word each in the expansion's LDS)
 constexpr u32 kMaxEff = 32;        // effects per schema the step applies (more set kStatusCapacity)
 
 /// The word offsets of a wave's LDS region: the view, the state row, then the uniform binding, the 64 lanes' bindings

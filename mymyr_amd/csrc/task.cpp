@@ -1957,6 +1957,10 @@ private:
         h.off_witness = any_witness ? put(witness.data(), witness.size() * sizeof(DevWitness)) : 0;
         h.lazy = lazy ? 1 : 0;
         h.simple = checks.empty() && C->label_width <= kLaneDepth + 1 ? 1 : 0;
+        h.listable = h.simple && n <= 0xFFFF ? 1 : 0;
+        for (const DevSchema& ds : schemas)
+            if (ds.eff_end - ds.eff_begin > kListEff)
+                h.listable = 0;
         std::memcpy(img.data(), &h, sizeof(h));
         C->image = std::move(img);
     }

@@ -249,6 +249,7 @@ struct DevStep
 
 constexpr u32 kMaxParams = 32;
 constexpr u32 kLaneDepth = 3;  // levels of a lane's nested count that the kernels unroll
+constexpr u32 kListEff = 6;    // effects of a listed successor (one register each)
 
 /// Per schema: plans P_j (j = 0..arity) count the bindings with parameters [0, j) bound; filters F_i (i < arity) give
 /// the candidates of parameter i with [0, i) bound (the lexicographic pick).
@@ -351,7 +352,7 @@ struct DevTaskHeader
     u32 init_count;     // successors of the initial state (filled once the device has counted them)
     u32 lazy;           // 1: lazy slots (slot_of, records, goal lists and initial row sized for every canonical atom)
     u32 simple;         // no checks, and every schema has at most kLaneDepth + 1 parameters
-    u32 pad;
+    u32 listable;       // simple, at most kListEff effects per schema, objects of 16 bits
     u64 off_deltas;     // DevDelta
     u64 off_witness;    // DevWitness per schema (0: no schema has a witness parameter)
 };

@@ -98,3 +98,37 @@ def test_pad_of_rows_at_any_alignment(k, shift):
         b = p["binding"][i].cpu().numpy()
         assert np.array_equal(b[:c], bind[off[i]: off[i] + c]) and (b[c:] == -1).all()
     assert [int(h) for h in x["succ_hash"].cpu().numpy().view(np.uint64)] == [port.hash_state(r) for r in succ.view(np.uint64)]
+
+
+@pytest.mark.parametrize("name", TASKS + ["crowded"])
+def test_expansion_equals_the_successor_listing(name, golden):
+    """The flat expansion lists successors 64 at a time from a list of 128 bindings (crowded: more than 128 successors
+    under one word of a first parameter; every arity, effect count and atom layout of the suite's tasks), the successor
+    listing enumerates them one by one: the same labels and rows, and the rows' flags follow from them."""
+    import torch
+
+    from mymyr_amd import gen, rl
+    from mymyr_amd.task import Task
+
+    t = Task.from_text(gen.transport(6, 16, 80, seed=3)) if name == "crowded" else Task.from_text_file(golden.task_path(name))
+    pool = rl.DeviceEnvPool(t, 37, seed=5, max_steps=None)
+    pool.reset()
+    for _ in range(9):
+        pool.step()
+    s = pool.states.clone()
+    x = rl.expand(t, s, goal=True, noops=True, hashes=True)
+    cap = int((x["offsets"][1:] - x["offsets"][:-1]).max())
+    count, schema, binding, rows = rl.successors(t, s, cap=max(cap, 1))
+    assert torch.equal(count, (x["offsets"][1:] - x["offsets"][:-1]))
+    live = torch.arange(max(cap, 1), device="cuda")[None, :] < count[:, None]
+    assert torch.equal(x["schema"], schema[live]) and torch.equal(x["binding"], binding[live]) and torch.equal(x["succ"], rows[live])
+    parent = torch.arange(37, device="cuda", dtype=torch.int32)[:, None].expand(live.shape)[live]
+    assert torch.equal(x["parent"], parent)
+    assert torch.equal(x["noop"] != 0, (x["succ"] == s[parent.long()]).all(dim=1))
+    d = rl.expand(t, s, drop_noops=True, noops=True)
+    keep = x["noop"] == 0
+    for i in range(37):
+        a, b = int(x["offsets"][i]), int(x["offsets"][i + 1])
+        if not keep[a:b].any():
+            keep[a:b] = True
+    assert torch.equal(d["succ"], x["succ"][keep]) and torch.equal(d["schema"], x["schema"][keep])
