@@ -497,7 +497,11 @@ __global__ __launch_bounds__(kLB) void k_ground_compact(StateSetView s, ParentRo
     constexpr int kBatch = 16;  // winners per group in flight (the list, record and row loads of each are independent)
     const u32 q = lane_id() % G;
     const u64 id0 = *size_now;
-    const u64 winners = min(m, *size_next - id0);
+    const u64 all = min(m, *size_next - id0);
+    // the winners past the limit are only reported, once (not with an atomic each on the one status word)
+    const u64 winners = min(all, limit > id0 ? limit - id0 : 0);
+    if (all > winners && blockIdx.x == 0 && threadIdx.x == 0)
+        atomicOr(status, kStatusCapacity);
     const u64 stride = static_cast<u64>(gridDim.x) * (kLB / G);
     // a grid sized for the whole chunk would mostly start waves that find no winner: a bounded grid strides instead
     for (u64 w0 = (static_cast<u64>(blockIdx.x) * kLB + threadIdx.x) / G; w0 < winners; w0 += kBatch * stride)
@@ -508,9 +512,7 @@ __global__ __launch_bounds__(kLB) void k_ground_compact(StateSetView s, ParentRo
         for (int b = 0; b < kBatch; ++b)
         {
             const u64 w = w0 + b * stride;
-            live[b] = w < winners && id0 + w < limit;
-            if (w < winners && id0 + w >= limit && q == 0)
-                atomicOr(status, kStatusCapacity);
+            live[b] = w < winners;
             pa[b] = live[b] ? list[w] : 0;
         }
 #pragma unroll

@@ -61,28 +61,47 @@ __global__ __launch_bounds__(kWB) void k_wide_compact(StateSetView s, const u64*
                                                      const u8* __restrict__ goal, u64 first, const u64* __restrict__ parent_ids,
                                                      u64* __restrict__ nodes, u8* __restrict__ goal_id, u32* __restrict__ status)
 {
+    // several winners of a group in flight: their list entries, then their rows, are independent loads 
+    constexpr int kBatch = K == 0 ? 1 : K >= 8 ? 1 : 8 / K;
     const u32 q = lane_id() % G;
     const u64 id0 = *size_now;
-    const u64 winners = min(m, *size_next - id0);
-    for (u64 w = (static_cast<u64>(blockIdx.x) * kWB + threadIdx.x) / G; w < winners; w += static_cast<u64>(gridDim.x) * (kWB / G))
+    const u64 all = min(m, *size_next - id0);
+    // the winners past the limit are only reported, once (an atomic each on the one status word took 2.4 ms where a search
+    // was cut inside a chunk of a million)
+    const u64 winners = min(all, limit > id0 ? limit - id0 : 0);
+    if (all > winners && blockIdx.x == 0 && threadIdx.x == 0)
+        atomicOr(status, kStatusCapacity);
+    const u64 stride = static_cast<u64>(gridDim.x) * (kWB / G);
+    for (u64 w0 = (static_cast<u64>(blockIdx.x) * kWB + threadIdx.x) / G; w0 < winners; w0 += kBatch * stride)
     {
-        const u64 id = id0 + w;
-        if (id >= limit)
+        u64 j[kBatch];
+        bool live[kBatch];
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b)
         {
-            if (q == 0)
-                atomicOr(status, kStatusCapacity);
-            continue;
+            const u64 w = w0 + b * stride;
+            live[b] = w < winners;
+            j[b] = live[b] ? list[w] : 0;
         }
-        const u64 j = list[w];
-        Slice<G, K> r;
-        load_row<G, K>(rows + j * s.words, s.words, q, r);
-        store_row<G, K>(s.arena + id * s.words, s.words, q, r);
-        if (q == 0)
+        Slice<G, K> r[kBatch];
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b)
+            if (live[b])
+                load_row<G, K>(rows + j[b] * s.words, s.words, q, r[b]);
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b)
         {
-            // parents gathered in an ordered layer's expansion order carry their ids in parent_ids
-            const u64 p = first + static_cast<u64>(parent[j]);
-            nodes[id] = ((parent_ids ? parent_ids[p] : p) << 32) | static_cast<u32>(index[j]);
-            goal_id[id] = goal[j];
+            if (!live[b])
+                continue;
+            const u64 id = id0 + w0 + b * stride;
+            store_row<G, K>(s.arena + id * s.words, s.words, q, r[b]);
+            if (q == 0)
+            {
+                // parents gathered in an ordered layer's expansion order carry their ids in parent_ids
+                const u64 p = first + static_cast<u64>(parent[j[b]]);
+                nodes[id] = ((parent_ids ? parent_ids[p] : p) << 32) | static_cast<u32>(index[j[b]]);
+                goal_id[id] = goal[j[b]];
+            }
         }
     }
 }

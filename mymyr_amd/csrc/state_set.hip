@@ -291,12 +291,18 @@ void with_shape(u32 W, F&& f)
         f.template operator()<4, 1>();
     else if (W <= 16)
         f.template operator()<4, 2>();  // four lanes of two pairs: faster than eight of one on 16-word rows
+    // sixteen lanes a row up to 256 words: four rows' probe chains (row, entry, compared row) in flight per wave where a
+    // wave per row waits for one (transport search, 176-word rows)
     else if (W <= 32)
         f.template operator()<16, 1>();
+    else if (W <= 64)
+        f.template operator()<16, 2>();
     else if (W <= 128)
-        f.template operator()<64, 1>();
+        f.template operator()<16, 4>();
+    else if (W <= 192)
+        f.template operator()<16, 6>();
     else if (W <= 256)
-        f.template operator()<64, 2>();
+        f.template operator()<16, 8>();
     else if (W <= 512)
         f.template operator()<64, 4>();
     else if (W <= 1024)

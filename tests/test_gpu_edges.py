@@ -132,3 +132,28 @@ def test_expansion_equals_the_successor_listing(name, golden):
         if not keep[a:b].any():
             keep[a:b] = True
     assert torch.equal(d["succ"], x["succ"][keep]) and torch.equal(d["schema"], x["schema"][keep])
+
+
+@pytest.mark.parametrize("words", [17, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257])
+def test_state_set_at_the_lane_group_shapes(words):
+    """Rows at the edges of the probe's lane-group shapes, with duplicates inside a batch and across batches: ids are
+    first-occurrence ranks."""
+    import torch
+
+    from mymyr_amd import hip
+
+    rng = np.random.default_rng(words)
+    base = rng.integers(0, 1 << 63, size=(700, words), dtype=np.uint64)
+    base[:, -1] &= np.uint64(rng.integers(0, 2))
+    pick = rng.integers(0, 700, size=2500)
+    rows = base[pick]
+    s = hip.StateSet(1024, words, 0.5, batch=1000)
+    first, want = {}, []
+    for p in pick:
+        want.append(first.setdefault(int(p), len(first)))
+    dev = torch.from_numpy(rows.view(np.int64)).cuda()
+    ids = torch.cat([s.insert(dev[:1700])[1], s.insert(dev[1700:])[1]]).cpu().numpy()
+    assert len(s) == len(first) and ids.tolist() == want
+    got = torch.from_dlpack(s.rows()).view(torch.int64).cpu().numpy().view(np.uint64)
+    order = [p for p, _ in sorted(first.items(), key=lambda x: x[1])]
+    assert np.array_equal(got, base[order])
