@@ -173,24 +173,13 @@ __device__ __forceinline__ u64 action_mask(const u64* B, const GroundDev& g, u64
     return B[rec & 0x7FFF] & B[(rec >> 16) & 0xFFFF] & B[(rec >> 32) & 0xFFFF] & B[rec >> 48];
 }
 
-// Successor counts and goal flags of parents [first, first + n): a wave takes 64 parents bit-sliced in LDS; each lane
-// tests one action of a group of 64 against all 64 parents at once (an AND of the action's precondition slot words),
-// and a transpose turns the group's masks into each parent's 64 action bits.
-template<int W>
-__global__ __launch_bounds__(kTW * kWave) void k_ground_count(const u64* __restrict__ arena, u64 first, u32 n, GroundDev g, GoalDev goal,
-                                                             u32* __restrict__ counts, u8* __restrict__ goal_flags)
+/// The wave's parents (bit mask over the slices B of its 64, the valid ones in vm) that are goal states.
+__device__ __forceinline__ u64 goal_parents(const u64* B, const GoalDev& goal, u64 vm)
 {
-    __shared__ u64 Bs[kTW][Slices<W>::kWords];
-    const u32 lane = lane_id(), wave = threadIdx.x / kWave;
-    const u32 base = (blockIdx.x * kTW + wave) * kWave;
-    if (base >= n)
-        return;
-    u64* B = Bs[wave];
-    const u64 vm = load_slices<W>(B, arena, first, base, n, lane);
-    u64 gm = 0;
     if (goal.any.any)
     {
         // AnyOf: the parents for which one of the goals holds, goal by goal over the bit slices
+        u64 gm = 0;
         for (u32 k = 0; k < goal.any.count; ++k)
         {
             u64 m = vm;
@@ -200,19 +189,25 @@ __global__ __launch_bounds__(kTW * kWave) void k_ground_count(const u64* __restr
                 m &= ~B[goal.any.slots[i]];
             gm |= m;
         }
+        return gm;
     }
-    else
-    {
-        gm = goal.unsat ? 0 : vm;
-        for (u32 i = 0; i < goal.npos; ++i)
-            gm &= B[goal.pos[i]];
-        for (u32 i = 0; i < goal.nneg; ++i)
-            gm &= ~B[goal.neg[i]];
-    }
-    // Per lane (one action of each group), a bit-sliced counter over the 64 parents: plane k holds bit k of how many of
-    // the lane's actions so far apply to each parent. Adding a group's mask is a ripple carry through the planes, and
-    // only the final planes are transposed (bit k of parent t's count over the lanes = popcount of plane k's column t),
-    // instead of one transpose per group. 64 groups at most between flushes keep every counter below 2^7.
+    u64 gm = goal.unsat ? 0 : vm;
+    for (u32 i = 0; i < goal.npos; ++i)
+        gm &= B[goal.pos[i]];
+    for (u32 i = 0; i < goal.nneg; ++i)
+        gm &= ~B[goal.neg[i]];
+    return gm;
+}
+
+/// How many of the actions [a0, a1) (multiples of 64) apply to the lane's parent, over the slices B of the wave's 64.
+///
+/// Per lane (one action of each group), a bit-sliced counter over the 64 parents: plane k holds bit k of how many of
+/// the lane's actions so far apply to each parent. Adding a group's mask is a ripple carry through the planes, and
+/// only the final planes are transposed (bit k of parent t's count over the lanes = popcount of plane k's column t),
+/// instead of one transpose per group. 64 groups at most between flushes keep every counter below 2^7.
+template<int W>
+__device__ __forceinline__ u32 count_actions(const u64* B, const GroundDev& g, u32 a0, u32 a1, u64 vm, u32 lane)
+{
     u64 plane[kCountPlanes] = {};
     u32 cnt = 0, groups = 0;
     auto add = [&](u64 m) {
@@ -233,8 +228,7 @@ __global__ __launch_bounds__(kTW * kWave) void k_ground_count(const u64* __restr
         }
         groups = 0;
     };
-    u32 a0 = 0;
-    for (; a0 + 4 * kWave <= g.num_padded; a0 += 4 * kWave)
+    for (; a0 + 4 * kWave <= a1; a0 += 4 * kWave)
     {
         // four independent groups in flight
         u64 m[4];
@@ -248,7 +242,7 @@ __global__ __launch_bounds__(kTW * kWave) void k_ground_count(const u64* __restr
         if (groups == 64)
             flush();
     }
-    for (; a0 < g.num_padded; a0 += kWave)
+    for (; a0 < a1; a0 += kWave)
     {
         const u32 a = a0 + lane;
         add(action_mask<W>(B, g, g.fast[a], a, vm));
@@ -256,6 +250,25 @@ __global__ __launch_bounds__(kTW * kWave) void k_ground_count(const u64* __restr
             flush();
     }
     flush();
+    return cnt;
+}
+
+// Successor counts and goal flags of parents [first, first + n): a wave takes 64 parents bit-sliced in LDS; each lane
+// tests one action of a group of 64 against all 64 parents at once (an AND of the action's precondition slot words),
+// and a transpose turns the groups' masks into each parent's count.
+template<int W>
+__global__ __launch_bounds__(kTW * kWave) void k_ground_count(const u64* __restrict__ arena, u64 first, u32 n, GroundDev g, GoalDev goal,
+                                                             u32* __restrict__ counts, u8* __restrict__ goal_flags)
+{
+    __shared__ u64 Bs[kTW][Slices<W>::kWords];
+    const u32 lane = lane_id(), wave = threadIdx.x / kWave;
+    const u32 base = (blockIdx.x * kTW + wave) * kWave;
+    if (base >= n)
+        return;
+    u64* B = Bs[wave];
+    const u64 vm = load_slices<W>(B, arena, first, base, n, lane);
+    const u64 gm = goal_parents(B, goal, vm);
+    const u32 cnt = count_actions<W>(B, g, 0, g.num_padded, vm, lane);
     const u32 t = base + lane;
     if (t < n)
     {
@@ -537,6 +550,209 @@ __global__ __launch_bounds__(kLB) void k_ground_compact(StateSetView s, ParentRo
     }
 }
 
+// Small layers, one block for several whole layers: a search over few states (a short plan, a search's first layers) is
+// bound by the launches and host round trips of a layer (17 launches and two synchronizations, over 100 us), not by its
+// few thousand successors. One block of 16 waves takes a layer through the same steps between barriers: counts (the
+// waves that share 64 parents split the actions, where a wave of k_ground_count takes all of them), offsets, records,
+// probes, ranks and rows. Its winners' entries are settled to their ids on the spot, so the layers share one epoch. A layer
+// that is not all plain is left untouched for the host's path: more than kSmallParents parents or kSmallLanes lanes of
+// successors, a goal state to stop at, the expansion budget ending inside it, or successors that could fill the store.
+//
+// Shortest path in a 32x32 grid (16 layers, 16-word rows) 2.69 -> 1.05 ms, all of a gripper task (36 layers, the smaller of
+// them here) 5.54 -> 3.89 ms, both with the plan's records read at once (plan_nodes); a search whose layers explode is as
+// before. The limit on lanes is eight rounds of probes of the block's threads.
+constexpr u32 kSmallThreads = 1024;
+constexpr u32 kSmallWaves = kSmallThreads / kWave;
+constexpr u32 kSmallGroups = 8;  // groups of 64 parents, bit-sliced in LDS
+constexpr u32 kSmallParents = kSmallGroups * kWave;
+constexpr u32 kSmallLanes = 8192;
+constexpr u32 kSmallLayers = 64;             // layers per launch (the host checks its stop conditions between launches)
+constexpr u32 kSmallActions = u32{1} << 22;  // a layer's successors are counted in 32 bits
+enum SmallOut : u32
+{
+    kSoLayers = 0,     // layers expanded
+    kSoSize = 1,       // stored states
+    kSoGoals = 2,      // goal states among the expanded ones
+    kSoFirstGoal = 3,  // the first of them (~0: none)
+    kSoStatus = 4,
+    kSoRows = 5,  // [layers][3]: {expanded, generated, new}
+    kSoWords = kSoRows + 3 * kSmallLayers,
+};
+
+struct SmallArgs
+{
+    u64 pos, size;       // the layer's first state and the stored states
+    u64 max_states;      // no layer starts at this many states
+    u64 limit;           // a layer whose successors could make this many states is left
+    u64 budget;          // states that may still be expanded
+    u32 layers;          // at most this many layers
+    u32 stop_at_goal;
+    u64* cand_slot;
+    u32* list;
+    u8* flags;
+    u64* nodes;
+    u64* size_now;
+    u32* status;
+    u64* out;
+};
+
+template<int W, bool kCE>
+__global__ __launch_bounds__(kSmallThreads) void k_small_layers(StateSetView s, ParentRows<W, kCE> src, u32* cand_pa, GroundDev g, GoalDev goal,
+                                                               SmallArgs a)
+{
+    constexpr int G = kGroup<W>, K = kPairs<W>;
+    __shared__ u64 Bs[kSmallGroups][Slices<W>::kWords];
+    __shared__ u64 goal_mask[kSmallGroups];
+    __shared__ u32 cnt[kSmallWaves][kWave];
+    __shared__ u32 offs[kSmallParents];
+    __shared__ u32 part[kSmallWaves + 1];
+    const u32 tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    const u32 q = lane % G, gbase = lane - q;
+    u64 pos = a.pos, size = a.size, expanded = 0, goals = 0, first_goal = ~u64{0};
+    u32 layers = 0;
+    while (layers < a.layers)
+    {
+        const u64 ln = size - pos;
+        if (ln == 0 || ln > kSmallParents || size >= a.max_states || expanded + ln > a.budget)
+            break;
+        const u32 n = static_cast<u32>(ln);
+        const u32 groups = (n + kWave - 1) / kWave;
+        u32 pg = 1;  // the waves' parent groups (a power of two); kSmallWaves / pg waves split a group's actions
+        while (pg < groups)
+            pg *= 2;
+        const u32 grp = wave & (pg - 1), split = wave / pg, splits = kSmallWaves / pg;
+        const bool have = grp < groups;
+        u64* B = Bs[have ? grp : 0];
+        const u32 t = grp * kWave + lane;
+        if (have && split == 0)
+        {
+            const u64 vm = load_slices<W>(B, s.arena, pos, grp * kWave, n, lane);
+            const u64 gm = goal_parents(B, goal, vm);
+            if (lane == 0)
+                goal_mask[grp] = gm;
+        }
+        __syncthreads();
+        const u32 per = (g.num_padded / kWave + splits - 1) / splits * kWave;
+        const u32 a0 = min(split * per, g.num_padded), a1 = min(a0 + per, g.num_padded);
+        {
+            const u32 c = have ? count_actions<W>(B, g, a0, a1, B[Slices<W>::kOneSlot], lane) : 0;
+            cnt[wave][lane] = have && t < n ? c : 0;
+        }
+        __syncthreads();
+        // thread t < pg * 64: parent t's successors
+        u32 c = 0;
+        if (tid < pg * kWave)
+            for (u32 k = 0; k < splits; ++k)
+                c += cnt[k * pg + wave][lane];
+        u32 m;
+        const u32 at = block_exclusive<kSmallThreads>(c, part, &m);
+        if (tid < pg * kWave)
+            offs[tid] = at;
+        u64 layer_goals = 0, layer_first = ~u64{0};
+        for (u32 k = groups; k-- > 0;)
+            if (const u64 gm = goal_mask[k])
+            {
+                layer_goals += static_cast<u64>(__popcll(gm));
+                layer_first = pos + k * kWave + static_cast<u32>(__builtin_ctzll(gm));
+            }
+        if (m > kSmallLanes / G || size + m >= a.limit || (a.stop_at_goal && layer_goals))
+            break;
+        __syncthreads();
+        if (have)
+        {
+            u32 k = offs[t];
+            for (u32 i = 0; i < split; ++i)
+                k += cnt[i * pg + grp][lane];
+            const u64 vm = B[Slices<W>::kOneSlot];
+            for (u32 b0 = a0; b0 < a1; b0 += 4 * kWave)
+            {
+                u64 mt[4];
+#pragma unroll
+                for (u32 i = 0; i < 4; ++i)
+                {
+                    const u32 act = b0 + i * kWave + lane;
+                    mt[i] = b0 + i * kWave < a1 ? action_mask<W>(B, g, g.fast[act], act, vm) : 0;
+                }
+#pragma unroll
+                for (u32 i = 0; i < 4; ++i)
+                    mt[i] = transpose64(mt[i], lane);
+#pragma unroll
+                for (u32 i = 0; i < 4; ++i)
+                    for (u64 x = t < n ? mt[i] : 0; x; x &= x - 1)
+                        cand_pa[k++] = (t << src.abits) | (b0 + i * kWave + static_cast<u32>(__builtin_ctzll(x)));
+            }
+        }
+        __syncthreads();
+        src.first = pos;
+        for (u32 j = tid / G; j < m; j += kSmallThreads / G)
+        {
+            Slice<G, K> me;
+            src.load(j, q, me);
+            const u64 h = group_set_hash<G, K>(me, q, gbase);
+            const ProbeResult r = probe_insert<G, K>(s, src, j, me, h, q, gbase, a.flags, a.status);
+            if (q == 0)
+            {
+                a.cand_slot[j] = r.cand_slot;
+                if (r.lose)
+                    a.flags[j] = 0;
+            }
+        }
+        __syncthreads();
+        // ranks: each thread's run of consecutive candidates (losers' flags back to 1 for the next batch)
+        const u32 run = (m + kSmallThreads - 1) / kSmallThreads;
+        const u32 j0 = min(tid * run, m), j1 = min(j0 + run, m);
+        u32 won = 0;
+        for (u32 j = j0; j < j1; ++j)
+            won += a.flags[j];
+        u32 winners;
+        u32 w = block_exclusive<kSmallThreads>(won, part, &winners);
+        for (u32 j = j0; j < j1; ++j)
+            if (a.flags[j])
+                a.list[w++] = j;
+            else
+                a.flags[j] = 1;
+        __syncthreads();
+        for (u32 v = tid / G; v < winners; v += kSmallThreads / G)
+        {
+            const u32 j = a.list[v], pa = cand_pa[j];
+            const u64 id = size + v;
+            Slice<G, K> r;
+            src.template load_pa<G, K>(pa, q, r);
+            store_row<G, K>(s.arena + id * W, W, q, r);
+            if (q == 0)
+            {
+                a.nodes[id] = ((pos + src.parent_of(pa)) << 32) | src.action_of(pa);
+                const u64 cs = a.cand_slot[j];  // a winner's: (tag << 32) | slot
+                __hip_atomic_store(s.table + static_cast<u32>(cs), (cs & 0xFFFFFFFF00000000ull) | (id + 1), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        if (tid == 0)
+        {
+            u64* row = a.out + kSoRows + 3 * layers;
+            row[0] = n;
+            row[1] = m;
+            row[2] = winners;
+        }
+        goals += layer_goals;
+        first_goal = first_goal == ~u64{0} ? layer_first : first_goal;
+        expanded += n;
+        pos += n;
+        size += winners;
+        ++layers;
+        __syncthreads();
+    }
+    if (tid == 0)
+    {
+        *a.size_now = size;
+        a.out[kSoLayers] = layers;
+        a.out[kSoSize] = size;
+        a.out[kSoGoals] = goals;
+        a.out[kSoFirstGoal] = first_goal;
+        a.out[kSoStatus] = *a.status;
+    }
+}
+
 /// The fast records and the delete / add masks of the ground actions (host).
 template<int W>
 void build_action_tables(const GroundActions& ga, std::vector<u64>& fast, std::vector<u64>& masks)
@@ -751,7 +967,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     // search nodes: per stored state its first discovery (parent id << 32 | ground action); the start state has none
     u64* nodes = b.alloc<u64>(cap_states, "search nodes");
     r.memory_bytes = set.v.capacity * 8 + cap_states * (R + 8) + chunk * (4 + 8 + 1 + 4) + layer_cap * (S * 4 + 1 + S * 8 + 8);
-    b.host = static_cast<u64*>(pinned_acquire(kSmall * sizeof(u64)));
+    b.host = static_cast<u64*>(pinned_acquire(std::max<size_t>(kSmall, kSoWords) * sizeof(u64)));
     enum
     {
         kGoalSum = 0,   // goal states among the layer's expanded parents
@@ -796,6 +1012,11 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     u64 pos = 0;                           // states expanded or passed (the reference's queue position)
     u64 seen_parents = 0, seen_cands = 0;  // counted so far (the successors-per-parent estimate)
     double new_rate = 1.0;                 // new states per candidate of the last confirmed chunk
+    // small layers in one block (k_small_layers), where nothing is asked of the host between layers; chunk: the batch
+    // buffers hold a small layer's successors
+    const bool small_layers = !ev.on && !blocked.capacity && !o.goal_test && !o.on_pass && !o.on_progress && !lorder.ordered() &&
+                              !lorder.limited() && chunk >= kSmallLanes && g.num_padded <= kSmallActions && max_chunk_parents >= kSmallParents;
+    u64* const d_small_out = small_layers ? b.alloc<u64>(kSoWords, "small layers") : nullptr;
     while (!stopped)
     {
         if (pos >= set.size)
@@ -818,6 +1039,60 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
         }
         if (r.layers == o.max_depth)
             break;
+        if (const u64 n = set.size - pos; small_layers && n <= kSmallParents && seen_cands * n <= seen_parents * (kSmallLanes / kGroup<W>))
+        {
+            SmallArgs a{};
+            a.pos = pos;
+            a.size = set.size;
+            a.max_states = o.max_states;
+            a.limit = cap_states;
+            a.budget = o.max_expanded - r.expanded;
+            a.layers = std::min(kSmallLayers, o.max_depth - r.layers);
+            a.stop_at_goal = o.stop_at_goal ? 1 : 0;
+            a.cand_slot = set.cand_slot;
+            a.list = set.list;
+            a.flags = set.flags;
+            a.nodes = nodes;
+            a.size_now = state_set_size_now(set);
+            a.status = set.d_status;
+            a.out = d_small_out;
+            tm.begin(kKOther);
+            state_set_begin_batch(set, stream);
+            if (g.ce_off)
+                hipLaunchKernelGGL((k_small_layers<W, true>), dim3(1), dim3(kSmallThreads), 0, stream, set.v,
+                                   ParentRows<W, true>{set.v.arena, pos, cand_pa, d_masks, abits, g.ce_off, g.ce_meta, g.ce_soff, g.ce_slots},
+                                   cand_pa, g, goal, a);
+            else
+                hipLaunchKernelGGL((k_small_layers<W, false>), dim3(1), dim3(kSmallThreads), 0, stream, set.v,
+                                   ParentRows<W, false>{set.v.arena, pos, cand_pa, d_masks, abits}, cand_pa, g, goal, a);
+            launch_check("small layers");
+            state_set_end_settled(set);
+            tm.end(kKOther, 0);
+            hip_check(hipMemcpyAsync(b.host, d_small_out, kSoWords * sizeof(u64), hipMemcpyDeviceToHost, stream), "read small layers");
+            hip_check(hipStreamSynchronize(stream), "sync");
+            if (b.host[kSoStatus] & kStatusTableFull)
+                throw std::length_error("mymyr_amd: brfs: state table full");
+            const u64 done = b.host[kSoLayers];
+            for (u64 k = 0; k < done; ++k)
+            {
+                const u64* c = b.host + kSoRows + 3 * k;
+                lc.push_back({c[0], c[1], c[2]});
+                pos += c[0];
+                r.expanded += c[0];
+                r.generated += c[1];
+                seen_parents += c[0];
+                seen_cands += c[1];
+                if (c[1])
+                    new_rate = static_cast<double>(c[2]) / static_cast<double>(c[1]);
+            }
+            r.layers += static_cast<u32>(done);
+            r.goal_states += b.host[kSoGoals];
+            if (r.first_goal < 0 && b.host[kSoFirstGoal] != ~u64{0})
+                r.first_goal = static_cast<i64>(b.host[kSoFirstGoal]);
+            set.size = b.host[kSoSize];
+            if (done)
+                continue;
+        }
         ++r.layers;
         const u64 layer_begin = pos, layer_end = set.size;
         const u64 ln = layer_end - layer_begin;
@@ -1181,17 +1456,8 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     {
         // the plan to the first goal state tested, from the node records (first discoveries), and that state's row
         std::vector<u32> rev;
-        for (u64 v = static_cast<u64>(r.first_goal);;)
-        {
-            u64 nd = 0;
-            hip_check(hipMemcpy(&nd, nodes + v, sizeof(u64), hipMemcpyDeviceToHost), "plan node");
-            if (nd == ~u64{0})
-                break;
+        for (const u64 nd : plan_nodes(nodes, static_cast<u64>(r.first_goal), r.layers, b, stream))
             rev.push_back(static_cast<u32>(nd));
-            v = nd >> 32;
-            if (rev.size() > r.layers)
-                throw std::logic_error("mymyr_amd: brfs: the node records of the goal state form no path to the start");
-        }
         const u32 L = ga.label_width;
         r.plan_width = L;
         for (auto it = rev.rbegin(); it != rev.rend(); ++it)

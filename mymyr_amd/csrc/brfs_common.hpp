@@ -218,6 +218,39 @@ struct Buffers
     }
 };
 
+// The node records on the path from state v back to the start, in that order: out[1 ..], their number in out[0] (more than
+// `most`: out[0] = most + 1). One thread follows the parents, a load after the other.
+__global__ void k_plan_nodes(const u64* __restrict__ nodes, u64 v, u64 most, u64* __restrict__ out)
+{
+    u64 n = 0;
+    for (;;)
+    {
+        const u64 nd = nodes[v];
+        if (nd == ~u64{0})
+            break;
+        if (++n > most)
+            break;
+        out[n] = nd;
+        v = nd >> 32;
+    }
+    out[0] = n;
+}
+
+/// The node records ((parent id << 32) | action) from state `goal` back to the start, at most `most`: followed on
+/// the device and copied once, where a blocking copy per record is a host round trip per action of the plan.
+inline std::vector<u64> plan_nodes(const u64* nodes, u64 goal, u64 most, Buffers& b, hipStream_t stream)
+{
+    u64* const out = b.alloc<u64>(most + 1, "plan nodes");
+    hipLaunchKernelGGL(k_plan_nodes, dim3(1), dim3(1), 0, stream, nodes, goal, most, out);
+    launch_check("plan nodes");
+    std::vector<u64> path(most + 1);
+    hip_check(hipMemcpyAsync(path.data(), out, path.size() * sizeof(u64), hipMemcpyDeviceToHost, stream), "plan nodes");
+    hip_check(hipStreamSynchronize(stream), "plan nodes");
+    if (path[0] > most)
+        throw std::logic_error("mymyr_amd: brfs: the node records of the goal state form no path to the start");
+    return {path.begin() + 1, path.begin() + 1 + path[0]};
+}
+
 using Clock = std::chrono::steady_clock;
 
 /// The blocked states of a search on the device (BlockedView): the rows padded to the set's row width W, duplicates

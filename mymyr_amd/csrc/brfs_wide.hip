@@ -633,17 +633,8 @@ BrfsResultC brfs_wide(const CompiledTask& task, const TaskDev& dev, const BrfsOp
         // the plan from the node records: each names its parent and the successor's index in the parent's canonical
         // order; the label is that successor of the parent's expansion, generated again (brfs.cpp:1362-1388)
         std::vector<std::pair<u64, u32>> rev;
-        for (u64 v = static_cast<u64>(r.first_goal);;)
-        {
-            u64 nd = 0;
-            hip_check(hipMemcpy(&nd, nodes + v, sizeof(u64), hipMemcpyDeviceToHost), "plan node");
-            if (nd == ~u64{0})
-                break;
+        for (const u64 nd : plan_nodes(nodes, static_cast<u64>(r.first_goal), r.layers, b, stream))
             rev.push_back({nd >> 32, static_cast<u32>(nd)});
-            v = nd >> 32;
-            if (rev.size() > r.layers)
-                throw std::logic_error("mymyr_amd: brfs: the node records of the goal state form no path to the start");
-        }
         const u32 L = std::max<u32>(1, task.label_width);
         r.plan_width = L;
         u64* zero = b.alloc<u64>(1, "plan offset");

@@ -72,6 +72,9 @@ void state_set_sync(StateSet& s);
 inline u64* state_set_size_now(StateSet& s) { return s.d_size + s.cur; }
 inline u64* state_set_size_next(StateSet& s) { return s.d_size + (s.cur ^ 1); }
 inline void state_set_flip(StateSet& s) { s.cur ^= 1; }
+/// Ends a batch whose winners' entries were settled to their ids by its own kernel (and the size written in place): no
+/// entry holds the batch's epoch, so the next batch takes it again.
+inline void state_set_end_settled(StateSet& s) { --s.batches; }
 
 /// The winners of a batch of n candidates in order into s.list (losers' flags reset), their ids into the batch's
 /// epoch of id_map, is_new[j] (optional) the flags, and next size = size + winners.

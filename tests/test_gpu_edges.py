@@ -157,3 +157,26 @@ def test_state_set_at_the_lane_group_shapes(words):
     got = torch.from_dlpack(s.rows()).view(torch.int64).cpu().numpy().view(np.uint64)
     order = [p for p, _ in sorted(first.items(), key=lambda x: x[1])]
     assert np.array_equal(got, base[order])
+
+
+@pytest.mark.parametrize("name", ["gridworld", "gripper__prob05", "noop_switches", "witness_order_0", "blocks__probBLOCKS-8-0",
+                                  "sokoban-opt08-strips__p14", "strips"])
+def test_searches_by_small_layers_equal_the_launches(name, golden):
+    """Layers taken whole by one block and by the launches (a chunk too small for the block's batch): the same counts,
+    fingerprints, goal states and plans, with budgets of states, expansions and layers that end a search inside its small
+    layers, right after them and past them (layers of 1 to more than 512 parents)."""
+    from mymyr_amd import search
+    from mymyr_amd.task import Task
+
+    task = Task.from_text_file(golden.task_path(name))
+    cases = [dict(), dict(stop_at_goal=False)]
+    cases += [dict(stop_at_goal=False, max_states=n) for n in (1, 2, 5, 63, 64, 65, 500, 2000, 9000)]
+    cases += [dict(stop_at_goal=False, max_expanded=n) for n in (0, 1, 3, 64, 500, 513, 3000)]
+    cases += [dict(stop_at_goal=False, max_depth=n) for n in (0, 1, 3, 9)]
+    for kw in cases:
+        kw = {"max_states": 60000, **kw}
+        a = search.brfs(task, fingerprint=True, **kw)
+        b = search.brfs(task, fingerprint=True, chunk=2048, **kw)
+        key = lambda r: (r.status, r.states, r.expanded, r.generated, r.layers, r.num_goal_states, r.fingerprint, r.cost,  # noqa: E731
+                         [tuple(x) for x in r.layer_counts], [(x.schema, tuple(x.binding)) for x in r.plan])
+        assert key(a) == key(b), f"{name}: {kw}"
