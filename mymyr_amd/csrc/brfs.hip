@@ -34,6 +34,9 @@ constexpr int kTW = 4;        // waves per block of the per-parent kernels (64 p
 constexpr int kLB = 256;      // threads per block of the per-candidate kernels
 constexpr u64 kGeneral = 0x8000;  // fast-record flag: the action takes the general test
 constexpr u64 kStrideBlocks = 4096;  // grid of the grid-stride kernels (16 blocks of 256 threads per CU)
+// A search starts on 2^22 slots (32 MiB, 2^21 states) of its table and takes the whole of it when these fill: clearing the
+// table of the default 2^26 states (1.5 GiB) takes 0.27 ms, where many searches end within a few thousand states.
+constexpr u64 kStartSlots = u64{1} << 22;
 constexpr int kCountPlanes = 7;    // bit planes of the per-lane successor counters (counts up to 64 between flushes)
 
 struct GroundDev
@@ -923,7 +926,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
         throw std::invalid_argument("mymyr_amd: brfs: more than 2^25 - 1 ground actions");
     const u64 chunk = std::min<u64>(std::max<u64>(o.chunk ? o.chunk : kMaxBatch, ga.size() + 1), kMaxBatch);
     StateSet set;
-    state_set_create(set, cap_states, W, 0.5, chunk, stream, chunk);
+    state_set_create(set, cap_states, W, 0.5, chunk, stream, chunk, kStartSlots);
     struct SetGuard
     {
         StateSet& s;
@@ -966,7 +969,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     u64* small = b.alloc<u64>(kSmall, "scalars");
     // search nodes: per stored state its first discovery (parent id << 32 | ground action); the start state has none
     u64* nodes = b.alloc<u64>(cap_states, "search nodes");
-    r.memory_bytes = set.v.capacity * 8 + cap_states * (R + 8) + chunk * (4 + 8 + 1 + 4) + layer_cap * (S * 4 + 1 + S * 8 + 8);
+    r.memory_bytes = set.slots * 8 + cap_states * (R + 8) + chunk * (4 + 8 + 1 + 4) + layer_cap * (S * 4 + 1 + S * 8 + 8);
     b.host = static_cast<u64*>(pinned_acquire(std::max<size_t>(kSmall, kSoWords) * sizeof(u64)));
     enum
     {
@@ -1057,6 +1060,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             a.status = set.d_status;
             a.out = d_small_out;
             tm.begin(kKOther);
+            state_set_reserve(set, set.size + kSmallLayers * (kSmallLanes / kGroup<W>), stream);
             state_set_begin_batch(set, stream);
             if (g.ce_off)
                 hipLaunchKernelGGL((k_small_layers<W, true>), dim3(1), dim3(kSmallThreads), 0, stream, set.v,
@@ -1345,6 +1349,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
                 launch_check("ground emit");
                 tm.end(kKEmit, np * (R + 8) + m * 4);
                 tm.begin(kKInsert);
+                state_set_reserve(set, set.size + m, stream);
                 state_set_begin_batch(set, stream);
                 if (g.ce_off)
                     hipLaunchKernelGGL((k_ground_insert<W, true>), dim3(blocks_for(m * G, kLB)), dim3(kLB), 0, stream, set.v, src_ce, m,

@@ -225,6 +225,30 @@ __global__ void k_set_words(u64* p, u64 a, u64 b, u32* status)
     *status = 0;
 }
 
+// The rows [0, n) of the arena, all different, into the cleared table as settled entries.
+template<int G, int K>
+__global__ __launch_bounds__(kBlock) void k_enter_rows(StateSetView s, u64 n)
+{
+    u64 j;
+    u32 q, gbase;
+    group_of<G>(j, q, gbase);
+    if (j >= n)
+        return;
+    Slice<G, K> r;
+    load_row<G, K>(s.arena + j * s.words, s.words, q, r);
+    const u64 h = group_set_hash<G, K>(r, q, gbase);
+    if (q != 0)
+        return;
+    const u64 e = ((h >> 32) << 32) | (j + 1);
+    u64 slot = slot_of_hash(h, s.capacity);
+    for (u64 probes = 0; probes < s.capacity; ++probes)
+    {
+        if (atomicCAS(reinterpret_cast<unsigned long long*>(s.table + slot), 0ull, static_cast<unsigned long long>(e)) == 0)
+            return;
+        slot = slot + 1 == s.capacity ? 0 : slot + 1;
+    }
+}
+
 // The dedup stream: row i is, with probability `dup` (i > 0), an exact copy of row src(i) < i, else fresh words
 // mix64(seed + (16 i + k + 1) * gamma). Counter-based, so any range of rows is generated independently.
 constexpr u64 kGamma = 0x9E3779B97F4A7C15ULL;
@@ -379,7 +403,8 @@ void launch_hash_rows(const u64* rows, u64 n, u32 words, u64* out, hipStream_t s
     launch_check("hash_rows");
 }
 
-void state_set_create(StateSet& s, u64 max_states, u32 words, double max_load, u64 batch_cap, hipStream_t stream, u64 pending)
+void state_set_create(StateSet& s, u64 max_states, u32 words, double max_load, u64 batch_cap, hipStream_t stream, u64 pending,
+                      u64 start_slots)
 {
     if (words == 0)
         throw std::invalid_argument("mymyr_amd: state set rows need at least one word");
@@ -395,7 +420,9 @@ void state_set_create(StateSet& s, u64 max_states, u32 words, double max_load, u
     if (cap >= (u64{1} << 32) - 1)
         throw std::invalid_argument("mymyr_amd: state set table capacity above 2^32 - 2 slots");
     s.v.words = words;
-    s.v.capacity = cap;
+    s.v.capacity = start_slots && start_slots <= cap / 4 ? start_slots : cap;
+    s.slots = cap;
+    s.max_load = max_load;
     s.max_states = max_states;
     s.batch_cap = std::clamp<u64>(batch_cap, 1, kMaxBatch);
     // epochs in rotation: as many as fit 512 MiB of id maps (the 2^25-candidate batches of the BrFS: 64), at least 4
@@ -407,7 +434,7 @@ void state_set_create(StateSet& s, u64 max_states, u32 words, double max_load, u
     s.v.id_limit = s.id_limit;
     s.v.id_stride = blocks;
     s.v.max_rows = max_states;
-    s.v.table = dev_alloc<u64>(cap, "state set table");
+    s.v.table = dev_alloc<u64>(s.slots, "state set table");
     s.v.arena = dev_alloc<u64>(max_states * words, "state set arena");
     s.cand_slot = dev_alloc<u64>(s.batch_cap, "state set batch slots");
     s.flags = dev_alloc<u8>((s.batch_cap + 15) / 16 * 16, "state set batch flags");
@@ -453,6 +480,20 @@ void state_set_clear(StateSet& s, hipStream_t stream)
     s.batches = 0;
     s.v.epoch = 0;
     s.last = stream;
+}
+
+void state_set_reserve(StateSet& s, u64 states, hipStream_t stream)
+{
+    if (s.v.capacity == s.slots || static_cast<double>(states) <= static_cast<double>(s.v.capacity) * s.max_load)
+        return;
+    s.v.capacity = s.slots;
+    launch_fill_u32(reinterpret_cast<u32*>(s.v.table), s.v.capacity * 2, 0u, stream);
+    if (s.size)
+        with_shape(s.v.words, [&]<int G, int K>() {
+            hipLaunchKernelGGL((k_enter_rows<G, K>), dim3(group_blocks<G>(s.size)), dim3(kBlock), 0, stream, s.v, s.size);
+        });
+    launch_check("state set reserve");
+    s.batches = 0;  // no entry holds an epoch
 }
 
 void state_set_begin_batch(StateSet& s, hipStream_t stream)

@@ -41,13 +41,19 @@ struct StateSet
     u64* id_limit = nullptr;        // [epochs] the epochs' cut ids (v.id_limit)
     u32 epochs = 0;            // epochs in rotation (at most kMaxEpochs)
     u64 batches = 0;           // epochs taken since the last clear or settling pass
+    u64 slots = 0;             // slots of the table's allocation (v.capacity: those in use)
+    double max_load = 0;
 };
 
 /// Allocates a set for up to max_states rows of `words` words at the given maximum load: capacity =
 /// (max_states + pending) / load, where `pending` bounds the candidates a batch may hold as pending entries beyond
-/// max_states (a driver that cuts a batch at max_states after probing it).
+/// max_states (a driver that cuts a batch at max_states after probing it). With start_slots the set starts on that many of
+/// the table's slots where they are a small part of it, and the driver calls state_set_reserve before each batch.
 void state_set_create(StateSet& s, u64 max_states, u32 words, double max_load, u64 batch_cap, hipStream_t stream,
-                      u64 pending = 0);
+                      u64 pending = 0, u64 start_slots = 0);
+/// Makes room for `states` stored and pending states on a set that started on part of its table: past the slots in use,
+/// the whole table is taken and the stored rows [0, s.size) (s.size must be exact, no batch under way) enter it anew.
+void state_set_reserve(StateSet& s, u64 states, hipStream_t stream);
 /// Frees the set's device memory: with a stream, in that stream's order (the blocks are reused only after the work
 /// queued on it so far, which must include every use of the set); without one, after the device has finished all work.
 void state_set_destroy(StateSet& s, hipStream_t stream = nullptr);

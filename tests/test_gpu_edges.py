@@ -180,3 +180,21 @@ def test_searches_by_small_layers_equal_the_launches(name, golden):
         key = lambda r: (r.status, r.states, r.expanded, r.generated, r.layers, r.num_goal_states, r.fingerprint, r.cost,  # noqa: E731
                          [tuple(x) for x in r.layer_counts], [(x.schema, tuple(x.binding)) for x in r.plan])
         assert key(a) == key(b), f"{name}: {kw}"
+
+
+@pytest.mark.parametrize("props, max_states", [(60, (1 << 21) - 1), (60, (1 << 21) + 1), (200, 3000001), (640, 2500000)])
+def test_search_past_the_table_it_starts_on(props, max_states):
+    """A search takes its whole table when 2^21 states and a chunk's successors no longer fit half of the slots it started
+    on: chunks of several sizes reach that with different states stored, and store the same ones."""
+    from mymyr_amd import gen, search
+    from mymyr_amd.task import Task
+
+    task = Task.from_text(gen.random_strips(props, 2048, init_atoms=props // 8, seed=9), "dense")
+    kw = dict(max_states=max_states, stop_at_goal=False, fingerprint=True)
+    whole = search.brfs(task, **kw)
+    for chunk in (1 << 16, 1 << 20):
+        r = search.brfs(task, chunk=chunk, **kw)
+        assert (r.states, r.expanded, r.generated, r.fingerprint, r.layer_counts) == (whole.states, whole.expanded, whole.generated,
+                                                                                      whole.fingerprint, whole.layer_counts)
+    larger = search.brfs(task, **{**kw, "max_states": 1 << 25, "max_depth": len(whole.layer_counts) - 1})
+    assert larger.layer_counts == whole.layer_counts[:-1]
