@@ -37,7 +37,27 @@ constexpr u64 kStrideBlocks = 4096;  // grid of the grid-stride kernels (16 bloc
 // A search starts on 2^22 slots (32 MiB, 2^21 states) of its table and takes the whole of it when these fill: clearing the
 // table of the default 2^26 states (1.5 GiB) takes 0.27 ms, where many searches end within a few thousand states.
 constexpr u64 kStartSlots = u64{1} << 22;
+constexpr u32 kSmallActions = u32{1} << 22;  // at most this many: the successors of 512 parents are counted in 32 bits
 constexpr int kCountPlanes = 7;    // bit planes of the per-lane successor counters (counts up to 64 between flushes)
+
+/// The driver's device scalars (`small`) and their pinned mirror.
+enum GroundScalar : int
+{
+    kGoalSum = 0,   // goal states among the layer's expanded parents
+    kFirstGoal = 1, // first goal flag of a counted block
+    kChunkP = 2,    // chunk end parent, then its offset
+    kChunkOff = 3,
+    kSizeNow = 4,   // the set's size before the chunk's insert, then after it
+    kSizeNext = 8,
+    kChunkGoal = 10,  // goal states among a chunk's parents (read at the synchronization that confirms the chunk)
+    kSpare = 9,     // the capacity status of a cut chunk's compaction (expected there, not an error)
+    kCut = 5,       // the candidate of the state that fills the store
+    kBlockTotal = 6,
+    kFingerprint = 7,
+    kChunkPruned = 11,  // blocked candidates of a chunk (read at the synchronization that confirms it)
+    kBlockGoals = 13,   // goal states among the parents of a layer counted at once
+    kCutPruned = 12,    // blocked candidates of a cut chunk up to the cut
+};
 
 struct GroundDev
 {
@@ -367,6 +387,147 @@ __global__ __launch_bounds__(kTW * kWave) void k_ground_emit(const u64* __restri
     }
 }
 
+// The driver's scalars into their pinned mirror (one thread each; read once the stream has drained, without a copy of
+// its own), with the set's current size and status and, where given, a counted block's offset total.
+__global__ void k_scalars_to_host(const u64* __restrict__ small, const u64* __restrict__ size_now, const u32* __restrict__ status,
+                                  const u64* __restrict__ total, u64* __restrict__ host)
+{
+    const int i = static_cast<int>(threadIdx.x);
+    if (i < kSmall)
+        host[i] = i == kSizeNow ? *size_now : i == kCut ? *status : (i == kBlockTotal && total) ? *total : small[i];
+}
+
+// What follows the counts of a layer of at most kLayerParents parents, in one block and one launch: the successors'
+// offsets and total, the first goal state and the goal states' number, the chunk's end (as k_chunk_end) and the set's size and
+// status, the scalars straight into the pinned mirror. Launch by launch (three of the scan, the goal search's two, the
+// chunk's end, the gather and the copy) a layer of 10^4 parents spends longer in the gaps than in the kernels: all of a
+// gripper task, 26 such layers, 3.49 -> 2.05 ms with these in one. Each thread has its counts of all passes in flight at
+// once; a pass is 4,096 parents, four to a thread.
+constexpr u32 kLayerPasses = 8;
+constexpr u32 kLayerPass = 4 * 1024;
+constexpr u32 kLayerParents = kLayerPasses * kLayerPass;
+__global__ __launch_bounds__(1024) void k_layer_offsets(const u32* __restrict__ counts, const u8* __restrict__ goal_flags, u32 n,
+                                                        u64* __restrict__ offsets, u64 bound, const u64* __restrict__ size_now,
+                                                        const u32* __restrict__ status, u64* __restrict__ host)
+{
+    constexpr u32 kWaves = 1024 / kWave;
+    static_assert(kLayerPasses * kWaves == 2 * kWave, "two wave sums per lane of the first wave");
+    __shared__ u32 sums[kLayerPasses * kWaves];
+    __shared__ u64 before[kLayerPasses * kWaves + 1];
+    __shared__ u32 goal_first, goal_count;
+    const u32 tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+    if (tid == 0)
+    {
+        goal_first = ~u32{0};
+        goal_count = 0;
+    }
+    __syncthreads();
+    u32 v[kLayerPasses][4];
+    u32 first = ~u32{0}, goals = 0;
+#pragma unroll
+    for (u32 k = 0; k < kLayerPasses; ++k)
+    {
+        const u32 i = k * kLayerPass + 4 * tid;
+        u32 f = 0;
+        if (i + 4 <= n)
+        {
+            const uint4 x = *reinterpret_cast<const uint4*>(counts + i);
+            v[k][0] = x.x;
+            v[k][1] = x.y;
+            v[k][2] = x.z;
+            v[k][3] = x.w;
+            f = *reinterpret_cast<const u32*>(goal_flags + i);
+        }
+        else
+        {
+#pragma unroll
+            for (u32 e = 0; e < 4; ++e)
+            {
+                v[k][e] = i + e < n ? counts[i + e] : 0;
+                f |= (i + e < n ? static_cast<u32>(goal_flags[i + e]) : 0u) << (8 * e);
+            }
+        }
+#pragma unroll
+        for (u32 e = 0; e < 4; ++e)
+            if ((f >> (8 * e)) & 0xFF)
+            {
+                first = min(first, i + e);
+                ++goals;
+            }
+    }
+    if (goals)
+    {
+        atomicMin(&goal_first, first);
+        atomicAdd(&goal_count, goals);
+    }
+    u32 at[kLayerPasses];  // the counts before the thread's in its wave's run of the pass (at most 256 kSmallActions)
+#pragma unroll
+    for (u32 k = 0; k < kLayerPasses; ++k)
+    {
+        const u32 s = v[k][0] + v[k][1] + v[k][2] + v[k][3];
+        const u32 inc = wave_inclusive(s);
+        at[k] = inc - s;
+        if (lane == kWave - 1)
+            sums[k * kWaves + wave] = inc;
+    }
+    __syncthreads();
+    if (wave == 0)
+    {
+        const u64 x = sums[2 * lane], y = sums[2 * lane + 1];
+        const u64 inc = wave_inclusive64(x + y);
+        before[2 * lane] = inc - x - y;
+        before[2 * lane + 1] = inc - y;
+        if (lane == kWave - 1)
+            before[kLayerPasses * kWaves] = inc;
+    }
+    __syncthreads();
+#pragma unroll
+    for (u32 k = 0; k < kLayerPasses; ++k)
+    {
+        const u32 i = k * kLayerPass + 4 * tid;
+        const u64 o0 = before[k * kWaves + wave] + at[k], o1 = o0 + v[k][0], o2 = o1 + v[k][1], o3 = o2 + v[k][2];
+        if (i + 4 <= n)
+        {
+            *reinterpret_cast<ulonglong2*>(offsets + i) = ulonglong2{o0, o1};
+            *reinterpret_cast<ulonglong2*>(offsets + i + 2) = ulonglong2{o2, o3};
+        }
+        else
+        {
+            const u64 o[4] = {o0, o1, o2, o3};
+#pragma unroll
+            for (u32 e = 0; e < 4; ++e)
+                if (i + e < n)
+                    offsets[i + e] = o[e];
+        }
+    }
+    const u64 total = before[kLayerPasses * kWaves];
+    if (tid == 0)
+        offsets[n] = total;
+    __syncthreads();
+    if (tid == 0)
+    {
+        u32 a = 1, b = n + 1;  // the first parent in [1, n + 1) past the bound
+        if (total <= bound)
+            a = b;
+        while (a < b)
+        {
+            const u32 mid = a + (b - a) / 2;
+            if (offsets[mid] <= bound)
+                a = mid + 1;
+            else
+                b = mid;
+        }
+        const u32 p = max(a - 1, 1u);
+        host[kChunkP] = p;
+        host[kChunkOff] = total <= bound ? total : offsets[p];
+        host[kBlockTotal] = total;
+        host[kFirstGoal] = goal_count ? u64{goal_first} : ~u64{0};
+        host[kBlockGoals] = goal_count;
+        host[kSizeNow] = *size_now;
+        host[kCut] = *status;
+    }
+}
+
 /// The successor rows of (parent, action) records as the row source of the state set's probe and compaction:
 /// candidate c's row = (parent row & ~delete mask) | add mask, recomputed wherever it is needed (the probe compares a
 /// pending entry against it, the compaction writes it), so candidate rows are never stored before they are new states.
@@ -570,7 +731,6 @@ constexpr u32 kSmallGroups = 8;  // groups of 64 parents, bit-sliced in LDS
 constexpr u32 kSmallParents = kSmallGroups * kWave;
 constexpr u32 kSmallLanes = 8192;
 constexpr u32 kSmallLayers = 64;             // layers per launch (the host checks its stop conditions between launches)
-constexpr u32 kSmallActions = u32{1} << 22;  // a layer's successors are counted in 32 bits
 enum SmallOut : u32
 {
     kSoLayers = 0,     // layers expanded
@@ -971,22 +1131,9 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     u64* nodes = b.alloc<u64>(cap_states, "search nodes");
     r.memory_bytes = set.slots * 8 + cap_states * (R + 8) + chunk * (4 + 8 + 1 + 4) + layer_cap * (S * 4 + 1 + S * 8 + 8);
     b.host = static_cast<u64*>(pinned_acquire(std::max<size_t>(kSmall, kSoWords) * sizeof(u64)));
-    enum
-    {
-        kGoalSum = 0,   // goal states among the layer's expanded parents
-        kFirstGoal = 1, // first goal flag of a counted block
-        kChunkP = 2,    // chunk end parent, then its offset
-        kChunkOff = 3,
-        kSizeNow = 4,   // the set's size before the chunk's insert, then after it
-        kSizeNext = 8,
-        kChunkGoal = 10,  // goal states among a chunk's parents (read at the synchronization that confirms the chunk)
-        kSpare = 9,     // the capacity status of a cut chunk's compaction (expected there, not an error)
-        kCut = 5,       // the candidate of the state that fills the store
-        kBlockTotal = 6,
-        kFingerprint = 7,
-        kChunkPruned = 11,  // blocked candidates of a chunk (read at the synchronization that confirms it)
-        kCutPruned = 12,    // blocked candidates of a cut chunk up to the cut
-    };
+    void* host_dev = nullptr;  // the mirror as the device writes it
+    hip_check(hipHostGetDevicePointer(&host_dev, b.host, 0), "pinned mirror");
+    u64* const mirror = static_cast<u64*>(host_dev);
     auto set_small = [&](int idx, u64 v) { hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, stream, small + idx, v); };
     auto sync_small = [&] {
         hip_check(hipMemcpyAsync(b.host, small, kSmall * sizeof(u64), hipMemcpyDeviceToHost, stream), "read scalars");
@@ -1019,7 +1166,6 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     // buffers hold a small layer's successors
     const bool small_layers = !ev.on && !blocked.capacity && !o.goal_test && !o.on_pass && !o.on_progress && !lorder.ordered() &&
                               !lorder.limited() && chunk >= kSmallLanes && g.num_padded <= kSmallActions && max_chunk_parents >= kSmallParents;
-    u64* const d_small_out = small_layers ? b.alloc<u64>(kSoWords, "small layers") : nullptr;
     while (!stopped)
     {
         if (pos >= set.size)
@@ -1058,7 +1204,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             a.nodes = nodes;
             a.size_now = state_set_size_now(set);
             a.status = set.d_status;
-            a.out = d_small_out;
+            a.out = mirror;
             tm.begin(kKOther);
             state_set_reserve(set, set.size + kSmallLayers * (kSmallLanes / kGroup<W>), stream);
             state_set_begin_batch(set, stream);
@@ -1072,7 +1218,6 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             launch_check("small layers");
             state_set_end_settled(set);
             tm.end(kKOther, 0);
-            hip_check(hipMemcpyAsync(b.host, d_small_out, kSoWords * sizeof(u64), hipMemcpyDeviceToHost, stream), "read small layers");
             hip_check(hipStreamSynchronize(stream), "sync");
             if (b.host[kSoStatus] & kStatusTableFull)
                 throw std::length_error("mymyr_amd: brfs: state table full");
@@ -1145,6 +1290,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
         {
             bool live = false;
             u64 p0 = 0, np = 0, m = 0;
+            u64 goals = ~u64{0};  // goal states among its parents (~0: summed on the device, b.host[kChunkGoal])
         } pend;
         // an observed search's events of a confirmed chunk: parents [p0e, p0e + npe) and candidates [0, me)
         auto emit = [&](u64 p0e, u64 npe, u64 me) {
@@ -1244,15 +1390,16 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             emit(pend.p0, pend.np, pend.m);
             row[0] += pend.np;
             row[1] += pend.m;
-            layer_goals += b.host[kChunkGoal];
+            layer_goals += pend.goals != ~u64{0} ? pend.goals : b.host[kChunkGoal];
             if (blocked.capacity)
                 layer_pruned += b.host[kChunkPruned];
             return false;
         };
         auto read_state = [&](const u64* block_total = nullptr) {
-            hipLaunchKernelGGL(k_gather_small, dim3(1), dim3(1), 0, stream, small, int{kSizeNow}, state_set_size_now(set), int{kCut},
-                               set.d_status, int{kBlockTotal}, block_total);
-            launch_check("gather");
+            hipLaunchKernelGGL(k_scalars_to_host, dim3(1), dim3(kWave), 0, stream, small, state_set_size_now(set), set.d_status, block_total,
+                               mirror);
+            launch_check("scalars");
+            hip_check(hipStreamSynchronize(stream), "sync");
         };
         while (p0 < lim && !stopped)
         {
@@ -1261,6 +1408,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             // count ahead when the counted parents past p0 hold less than a full chunk (and the layer has more)
             const bool count_now = counted < lim && counted_total - base < chunk;
             u64 nb = 0;
+            bool at_once = false;  // the whole layer counted here, its offsets and scalars by k_layer_offsets
             if (count_now)
             {
                 const u64 est = seen_parents ? std::max<u64>(1, (seen_cands + seen_parents - 1) / seen_parents) : 1;
@@ -1273,20 +1421,36 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
                     custom_goal_flags(o, par + (pbase + counted) * W, nb, W, goal_flags + counted, stream);
                 tm.end(kKCount, nb * (R + 5));
                 tm.begin(kKOther);
-                launch_exclusive_scan(counts + counted * S, offsets + counted * S, nb * S, scan_scratch, offsets + (counted + nb) * S, stream,
-                                      counted ? offsets + counted * S : nullptr);
-                set_small(kFirstGoal, ~u64{0});
-                hipLaunchKernelGGL(k_first_u8, dim3(std::min<u64>(blocks_for(nb, 256), 4096)), dim3(256), 0, stream, goal_flags + counted, nb,
-                                   small + kFirstGoal);
-                launch_check("count scan");
+                at_once = counted == 0 && p0 == 0 && nb == lim && nb <= std::min<u64>(kLayerParents, max_chunk_parents) &&
+                          g.num_padded <= kSmallActions;
+                if (at_once)
+                {
+                    hipLaunchKernelGGL(k_layer_offsets, dim3(1), dim3(1024), 0, stream, counts, goal_flags, static_cast<u32>(nb), offsets, chunk,
+                                       state_set_size_now(set), set.d_status, mirror);
+                    launch_check("layer offsets");
+                }
+                else
+                {
+                    launch_exclusive_scan(counts + counted * S, offsets + counted * S, nb * S, scan_scratch, offsets + (counted + nb) * S,
+                                          stream, counted ? offsets + counted * S : nullptr);
+                    set_small(kFirstGoal, ~u64{0});
+                    hipLaunchKernelGGL(k_first_u8, dim3(std::min<u64>(blocks_for(nb, 256), 4096)), dim3(256), 0, stream, goal_flags + counted,
+                                       nb, small + kFirstGoal);
+                    launch_check("count scan");
+                }
                 tm.end(kKOther, 0);
             }
             // the chunk end over what is counted, and the pending chunk's outcome, in one synchronization
-            hipLaunchKernelGGL(k_chunk_end, dim3(1), dim3(1), 0, stream, offsets, S, p0, std::min({counted + nb, lim, p0 + max_chunk_parents}),
-                               base + chunk, small + kChunkP);
-            launch_check("chunk end");
-            read_state(count_now ? offsets + (counted + nb) * S : nullptr);
-            sync_small();
+            if (at_once)
+                hip_check(hipStreamSynchronize(stream), "sync");
+            else
+            {
+                hipLaunchKernelGGL(k_chunk_end, dim3(1), dim3(1), 0, stream, offsets, S, p0, std::min({counted + nb, lim, p0 + max_chunk_parents}),
+                                   base + chunk, small + kChunkP);
+                launch_check("chunk end");
+                read_state(count_now ? offsets + (counted + nb) * S : nullptr);
+            }
+            const u64 block_goals = at_once ? b.host[kBlockGoals] : ~u64{0};
             if (count_now)
             {
                 const u64 total = b.host[kBlockTotal];
@@ -1383,10 +1547,15 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
                     state_set_resolve_ids(set, ev.cand_slot, m, ev.ids, stream);
                 state_set_flip(set);
             }
-            // the chunk's goal states, read at the synchronization that confirms it
-            set_small(kChunkGoal, 0);
-            hipLaunchKernelGGL(k_sum_u8, dim3(std::min<u64>(blocks_for(np, 256), 1024)), dim3(256), 0, stream, goal_flags + p0, u64{np},
-                               small + kChunkGoal);
+            // the chunk's goal states: those of a layer counted at once, none before the first, else read at the
+            // synchronization that confirms the chunk
+            const u64 goals = p1 <= first_goal ? 0 : (at_once && np == nb) ? block_goals : ~u64{0};
+            if (goals == ~u64{0})
+            {
+                set_small(kChunkGoal, 0);
+                hipLaunchKernelGGL(k_sum_u8, dim3(std::min<u64>(blocks_for(np, 256), 1024)), dim3(256), 0, stream, goal_flags + p0, u64{np},
+                                   small + kChunkGoal);
+            }
             if (blocked.capacity)
             {
                 set_small(kChunkPruned, 0);
@@ -1394,7 +1563,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
                     hipLaunchKernelGGL(k_sum_u8, dim3(std::min<u64>(blocks_for(m, 256), 1024)), dim3(256), 0, stream, blocked.hit, m,
                                        small + kChunkPruned);
             }
-            pend = Pending{true, p0, np, m};
+            pend = Pending{true, p0, np, m, goals};
             p0 = p1;
             base = end_off;
             if (p0 >= lim)
@@ -1403,7 +1572,6 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
         if (!stopped && pend.live)
         {
             read_state();
-            sync_small();
             confirm(b.host[kSizeNow], static_cast<u32>(b.host[kCut]));
         }
         if (halt.why)

@@ -26,6 +26,8 @@ namespace
 __global__ void k_chunk_end(const u64* __restrict__ offsets, u32 stride, u64 p0, u64 hi, u64 bound, u64* __restrict__ out)
 {
     u64 a = p0 + 1, b = hi + 1;  // the first parent in [p0 + 1, hi + 1) past the bound
+    if (hi > p0 && offsets[hi * stride] <= bound)
+        a = b;  // mostly: all of them fit (one load where the search is a chain of them)
     while (a < b)
     {
         const u64 mid = a + (b - a) / 2;
