@@ -387,28 +387,18 @@ __global__ __launch_bounds__(kTW * kWave) void k_ground_emit(const u64* __restri
     }
 }
 
-// The driver's scalars into their pinned mirror (one thread each; read once the stream has drained, without a copy of
-// its own), with the set's current size and status and, where given, a counted block's offset total.
-__global__ void k_scalars_to_host(const u64* __restrict__ small, const u64* __restrict__ size_now, const u32* __restrict__ status,
-                                  const u64* __restrict__ total, u64* __restrict__ host)
-{
-    const int i = static_cast<int>(threadIdx.x);
-    if (i < kSmall)
-        host[i] = i == kSizeNow ? *size_now : i == kCut ? *status : (i == kBlockTotal && total) ? *total : small[i];
-}
-
 // What follows the counts of a layer of at most kLayerParents parents, in one block and one launch: the successors'
 // offsets and total, the first goal state and the goal states' number, the chunk's end (as k_chunk_end) and the set's size and
-// status, the scalars straight into the pinned mirror. Launch by launch (three of the scan, the goal search's two, the
+// status into the driver's scalars. Launch by launch (three of the scan, the goal search's two, the
 // chunk's end, the gather and the copy) a layer of 10^4 parents spends longer in the gaps than in the kernels: all of a
-// gripper task, 26 such layers, 3.49 -> 2.05 ms with these in one. Each thread has its counts of all passes in flight at
+// gripper task, 26 such layers, 3.49 -> 2.25 ms with these in one. Each thread has its counts of all passes in flight at
 // once; a pass is 4,096 parents, four to a thread.
 constexpr u32 kLayerPasses = 8;
 constexpr u32 kLayerPass = 4 * 1024;
 constexpr u32 kLayerParents = kLayerPasses * kLayerPass;
 __global__ __launch_bounds__(1024) void k_layer_offsets(const u32* __restrict__ counts, const u8* __restrict__ goal_flags, u32 n,
                                                         u64* __restrict__ offsets, u64 bound, const u64* __restrict__ size_now,
-                                                        const u32* __restrict__ status, u64* __restrict__ host)
+                                                        const u32* __restrict__ status, u64* __restrict__ small)
 {
     constexpr u32 kWaves = 1024 / kWave;
     static_assert(kLayerPasses * kWaves == 2 * kWave, "two wave sums per lane of the first wave");
@@ -518,13 +508,13 @@ __global__ __launch_bounds__(1024) void k_layer_offsets(const u32* __restrict__ 
                 b = mid;
         }
         const u32 p = max(a - 1, 1u);
-        host[kChunkP] = p;
-        host[kChunkOff] = total <= bound ? total : offsets[p];
-        host[kBlockTotal] = total;
-        host[kFirstGoal] = goal_count ? u64{goal_first} : ~u64{0};
-        host[kBlockGoals] = goal_count;
-        host[kSizeNow] = *size_now;
-        host[kCut] = *status;
+        small[kChunkP] = p;
+        small[kChunkOff] = total <= bound ? total : offsets[p];
+        small[kBlockTotal] = total;
+        small[kFirstGoal] = goal_count ? u64{goal_first} : ~u64{0};
+        small[kBlockGoals] = goal_count;
+        small[kSizeNow] = *size_now;
+        small[kCut] = *status;
     }
 }
 
@@ -1131,9 +1121,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
     u64* nodes = b.alloc<u64>(cap_states, "search nodes");
     r.memory_bytes = set.slots * 8 + cap_states * (R + 8) + chunk * (4 + 8 + 1 + 4) + layer_cap * (S * 4 + 1 + S * 8 + 8);
     b.host = static_cast<u64*>(pinned_acquire(std::max<size_t>(kSmall, kSoWords) * sizeof(u64)));
-    void* host_dev = nullptr;  // the mirror as the device writes it
-    hip_check(hipHostGetDevicePointer(&host_dev, b.host, 0), "pinned mirror");
-    u64* const mirror = static_cast<u64*>(host_dev);
+    u64* const d_small_out = b.alloc<u64>(kSoWords, "small layers");
     auto set_small = [&](int idx, u64 v) { hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, stream, small + idx, v); };
     auto sync_small = [&] {
         hip_check(hipMemcpyAsync(b.host, small, kSmall * sizeof(u64), hipMemcpyDeviceToHost, stream), "read scalars");
@@ -1204,7 +1192,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             a.nodes = nodes;
             a.size_now = state_set_size_now(set);
             a.status = set.d_status;
-            a.out = mirror;
+            a.out = d_small_out;
             tm.begin(kKOther);
             state_set_reserve(set, set.size + kSmallLayers * (kSmallLanes / kGroup<W>), stream);
             state_set_begin_batch(set, stream);
@@ -1218,6 +1206,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             launch_check("small layers");
             state_set_end_settled(set);
             tm.end(kKOther, 0);
+            hip_check(hipMemcpyAsync(b.host, d_small_out, kSoWords * sizeof(u64), hipMemcpyDeviceToHost, stream), "read small layers");
             hip_check(hipStreamSynchronize(stream), "sync");
             if (b.host[kSoStatus] & kStatusTableFull)
                 throw std::length_error("mymyr_amd: brfs: state table full");
@@ -1396,10 +1385,10 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             return false;
         };
         auto read_state = [&](const u64* block_total = nullptr) {
-            hipLaunchKernelGGL(k_scalars_to_host, dim3(1), dim3(kWave), 0, stream, small, state_set_size_now(set), set.d_status, block_total,
-                               mirror);
-            launch_check("scalars");
-            hip_check(hipStreamSynchronize(stream), "sync");
+            hipLaunchKernelGGL(k_gather_small, dim3(1), dim3(1), 0, stream, small, int{kSizeNow}, state_set_size_now(set), int{kCut},
+                               set.d_status, int{kBlockTotal}, block_total);
+            launch_check("gather");
+            sync_small();
         };
         while (p0 < lim && !stopped)
         {
@@ -1426,7 +1415,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
                 if (at_once)
                 {
                     hipLaunchKernelGGL(k_layer_offsets, dim3(1), dim3(1024), 0, stream, counts, goal_flags, static_cast<u32>(nb), offsets, chunk,
-                                       state_set_size_now(set), set.d_status, mirror);
+                                       state_set_size_now(set), set.d_status, small);
                     launch_check("layer offsets");
                 }
                 else
@@ -1442,7 +1431,7 @@ BrfsResultC run(const CompiledTask& task, const BrfsTables& tb, const BrfsOption
             }
             // the chunk end over what is counted, and the pending chunk's outcome, in one synchronization
             if (at_once)
-                hip_check(hipStreamSynchronize(stream), "sync");
+                sync_small();
             else
             {
                 hipLaunchKernelGGL(k_chunk_end, dim3(1), dim3(1), 0, stream, offsets, S, p0, std::min({counted + nb, lim, p0 + max_chunk_parents}),
