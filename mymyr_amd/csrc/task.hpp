@@ -250,6 +250,7 @@ struct DevStep
 constexpr u32 kMaxParams = 32;
 constexpr u32 kLaneDepth = 3;  // levels of a lane's nested count that the kernels unroll
 constexpr u32 kListEff = 6;    // effects of a listed successor (one register each)
+constexpr u32 kListRegs = 4;  // words of a listed successor's row per lane kept in registers (rows up to 256 words)
 
 /// Per schema: plans P_j (j = 0..arity) count the bindings with parameters [0, j) bound; filters F_i (i < arity) give
 /// the candidates of parameter i with [0, i) bound (the lexicographic pick).
