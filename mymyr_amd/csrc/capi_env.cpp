@@ -44,7 +44,8 @@ struct mya_env
     SamplerDev sampler{};          // the instance sampler (instances 0: off)
     u32* d_thresholds = nullptr;   // device [m - 1]
     i32* d_indices = nullptr;      // device [m]
-    u32 wave_words = 0;  // LDS words per wave of the env's launches
+    u32 wave_words = 0;  // LDS words per wave of the env's expansions
+    u32 step_words = 0;  // and of its steps and counts
     u32 general = 0;     // some instance is not simple
     u64 sampled_rows = 0;
     i32* d_sampled = nullptr;  // [sampled_rows]: the sampled next instances of a step
@@ -153,7 +154,7 @@ void run_count(mya_env* env, const mya_env_batch* batch, CountArgs& a, hipStream
     a.status = env->d_status;
     a.cache_width = env->cache_width();
     a.mask_width = env->num_schemas;
-    a.wave_words = env->wave_words;
+    a.wave_words = env->step_words;
     a.general = env->general;
     launch_env_count(a, s);
 }
@@ -392,7 +393,8 @@ void create_env(mya_task* const* tasks, uint32_t count, const mya_env_config* co
             std::vector<const TaskDev*> all;
             for (const EnvInstance& in : e->inst)
                 all.push_back(&in.T);
-            e->wave_words = env_wave_words(all.data(), count);
+            e->wave_words = env_wave_words(all.data(), count, false);
+            e->step_words = env_wave_words(all.data(), count, true);
         }
         const u32 S = e->num_schemas, cw = e->cache_width();
         e->d_status = dev_alloc<u32>(1, "env status");
@@ -650,7 +652,7 @@ void env_step(mya_env* env, const mya_env_batch* batch, const mya_step_outputs* 
             launch_env_sample_next(env->sampler, env->d_seed, batch->first_env, batch->rows, batch->reset_counts, batch->sampling_seeds,
                                    batch->env_ids, const_cast<i32*>(a.next_task_ids), s);
         }
-        a.wave_words = env->wave_words;
+        a.wave_words = env->step_words;
         a.general = env->general;
         if (a.instances == 1)
         {
@@ -708,7 +710,7 @@ int mya_env_reserve(mya_env* env, uint64_t rows)
         if (rows == 0)
             return;
         scratch_rows(env, rows, &mya_env::d_sampled, &mya_env::sampled_rows);
-        prepare_env_launches(env->wave_words, env->general, env->instances() == 1);
+        prepare_env_launches(env->step_words, env->general, env->instances() == 1);
     });
 }
 

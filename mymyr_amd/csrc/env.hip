@@ -483,13 +483,13 @@ unsigned device_cus()
     return n;
 }
 
-u32 env_wave_words(const TaskDev* const* tasks, u32 n)
+u32 env_wave_words(const TaskDev* const* tasks, u32 n, bool step)
 {
     u32 words = 0;
     for (u32 k = 0; k < n; ++k)
     {
         check_schemas(*tasks[k]);
-        words = std::max(words, tasks[k]->l_words);
+        words = std::max(words, step ? tasks[k]->l_step : tasks[k]->l_words);
     }
     size_t lds = 0;
     block_shape(static_cast<size_t>(words) * 8, &lds);  // throws where a wave's region does not fit a workgroup
@@ -499,12 +499,12 @@ u32 env_wave_words(const TaskDev* const* tasks, u32 n)
 namespace
 {
 /// The LDS words per wave of a launch: given (a table's widest instance), or those of its one instance.
-u32 wave_words_of(u32 given, const TaskDev& T)
+u32 wave_words_of(u32 given, const TaskDev& T, bool step)
 {
     if (given)
         return given;
     const TaskDev* t = &T;
-    return env_wave_words(&t, 1);
+    return env_wave_words(&t, 1, step);
 }
 
 /// The kernels for simple tasks (TaskDev::simple; every instance of a table), or for any.
@@ -524,7 +524,7 @@ void launch_env_step(const EnvArgs& args, hipStream_t stream)
     if (args.rows == 0)
         return;
     EnvArgs a = args;
-    a.wave_words = wave_words_of(a.wave_words, a.T);
+    a.wave_words = wave_words_of(a.wave_words, a.T, true);
     size_t lds = 0;
     const unsigned nw = block_shape(static_cast<size_t>(a.wave_words) * 8, &lds);
     const bool visited = a.visited.capacity || a.revisited;
@@ -541,7 +541,7 @@ void launch_env_count(const CountArgs& args, hipStream_t stream)
     if (args.rows == 0)
         return;
     CountArgs a = args;
-    a.wave_words = wave_words_of(a.wave_words, a.T);
+    a.wave_words = wave_words_of(a.wave_words, a.T, true);
     size_t lds = 0;
     const unsigned nw = block_shape(static_cast<size_t>(a.wave_words) * 8, &lds);
     const EnvKernels k = kernels_for(a.T.simple && !a.general);
@@ -589,7 +589,7 @@ void launch_expand(const ExpandArgs& args, hipStream_t stream)
     if (args.rows == 0)
         return;
     ExpandArgs a = args;
-    a.wave_words = wave_words_of(a.wave_words, a.T);
+    a.wave_words = wave_words_of(a.wave_words, a.T, false);
     const bool simple = a.T.simple && !a.general;
     // successors 64 at a time, where every instance is listable and the call asks for whole rows (rows narrower than the
     // task's need their trimmed lengths, a successor at a time)

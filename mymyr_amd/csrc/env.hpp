@@ -157,8 +157,9 @@ void launch_env_count(const TaskDev& T, const u64* states, u64 rows, u32 words, 
                       hipStream_t stream, const u64* goal_pos = nullptr, const u64* goal_neg = nullptr, u32* status = nullptr,
                       u32 instance = 0, u32 schemas = 0);
 
-/// The LDS words per wave of launches over the instances (their largest); throws for an instance the kernels cannot take.
-u32 env_wave_words(const TaskDev* const* tasks, u32 n);
+/// The LDS words per wave of launches over the instances (their largest; step: of steps and counts, which need no enumeration
+/// scratch); throws for an instance the kernels cannot take.
+u32 env_wave_words(const TaskDev* const* tasks, u32 n, bool step);
 /// Raises the dynamic LDS limits of the step and count kernels of an env of one instance (`one`) or several, so that later
 /// launches make no runtime call besides the launch (HIP graph capture).
 void prepare_env_launches(u32 wave_words, bool general, bool one);

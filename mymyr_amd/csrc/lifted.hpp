@@ -40,7 +40,7 @@ struct TaskDev
     u32 listable;  // simple, at most kListEff effects per schema and objects of 16 bits: successors are listed (expand_listed)
     u32 lazy;      // lazy slots: an added atom without a slot is recorded in `missing`
     u64* missing;  // lazy slots: bit per canonical fluent atom (device; set by the successor kernels), else null
-    u32 l_row, l_dfs_m, l_ub, l_bind, l_counts, l_dfs_w, l_eff, l_before, l_cur, l_words;  // a wave's LDS region (set_region)
+    u32 l_row, l_dfs_m, l_ub, l_bind, l_counts, l_dfs_w, l_eff, l_before, l_cur, l_step, l_words;  // a wave's LDS region (set_region)
     const DevWitness* witness;  // per schema its witness parameters and plans (null: no schema has a witness)
 };
 
@@ -52,8 +52,11 @@ constexpr u32 kListCap = 128;      // successors listed at a time (a word each i
 constexpr u32 kMaxEff = 32;        // effects per schema the step applies (more set kStatusCapacity)
 
 /// The word offsets of a wave's LDS region: the view, the state row, then the uniform binding, the 64 lanes' bindings
-/// (A = the largest schema arity, at least 1), the per-schema counts, the successor enumeration's level cursors (A
-/// masks, A words), the effect scratch, and for plans deeper than kLaneDepth the lanes' enumeration cursors.
+/// (A = the largest schema arity, at least 1), the per-schema counts, for plans deeper than kLaneDepth the lanes'
+/// enumeration cursors (so far l_step words: the step's and the count's region), the successor enumeration's level
+/// cursors (A masks, A words) and its effect scratch. A step's region is what limits the waves of wide states: a
+/// transport_xl wave takes 22,824 bytes without the enumeration's scratch and 23,120 with it, seven waves to a CU or six
+/// (the allocation's granularity rounds the latter up past a seventh of the 160 KiB): 6.21 -> 5.38 ms per step.
 inline void set_region(TaskDev& t)
 {
     const u32 A = t.label_width ? t.label_width : 1;
@@ -64,14 +67,15 @@ inline void set_region(TaskDev& t)
         return at;
     };
     t.l_row = next(t.W);
-    t.l_dfs_m = next(A);
     t.l_ub = next((A + 1) / 2);
     t.l_bind = next(32 * A);
     t.l_counts = next((t.num_schemas + 1) / 2);
+    t.l_cur = next(A > kLaneDepth ? 64 * A + 32 * A : 0);
+    t.l_step = (w + 2) & ~1u;  // a word past the end: reads of two words at a bit position stay inside
+    t.l_dfs_m = next(A);
     t.l_dfs_w = next((A + 1) / 2);
     t.l_eff = next(kMaxEff / 2);
     t.l_before = next(kMaxEff / 2);
-    t.l_cur = next(A > kLaneDepth ? 64 * A + 32 * A : 0);
-    t.l_words = (w + 2) & ~1u;  // a word past the end: reads of two words at a bit position stay inside
+    t.l_words = (w + 2) & ~1u;
 }
 }  // namespace mya
