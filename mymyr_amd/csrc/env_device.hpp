@@ -179,14 +179,13 @@ __device__ __forceinline__ u64 cand_word(const Tab& H, const Lds& L, const DevSt
         else
         {
             // 64 bits from bit `rel` of the row on, those outside the row cleared
-            const i32 rel = c.delta + 64 * static_cast<i32>(w);
-            const u32 pos = at + static_cast<u32>(rel > 0 ? rel : 0), sh = pos & 63;
+            const RowBits b = row_bits(c, w);
+            const u32 pos = at + b.skip, sh = pos & 63;
             const auto r = L.view + (pos >> 6);
             v = (r[0] >> sh) | ((r[1] << 1) << (63 - sh));
-            const i32 keep = static_cast<i32>(c.stride) - (rel > 0 ? rel : 0);
-            v = keep >= 64 ? v : keep > 0 ? v & ((u64{1} << keep) - 1) : 0;
-            if (c.delta < 0 && rel < 0)
-                v = rel > -64 ? v << -rel : 0;
+            v = b.keep >= 64 ? v : b.keep > 0 ? v & ((u64{1} << b.keep) - 1) : 0;
+            if (c.delta < 0 && b.rel < 0)
+                v = b.rel > -64 ? v << -b.rel : 0;
         }
         if (c.rows != kNone)
             v = in ? v : 0;

@@ -209,6 +209,22 @@ struct DevTerm
     i32 delta;
 };
 
+/// Where window word w of a Bits term falls: the window word's first bit is bit `rel` of the row (negative: the row starts
+/// inside or after the word), its bits are read from bit `skip` of the row on, and the first `keep` of them are the row's
+/// (none if not positive). A parameter's window may be far longer than a row, and the last row ends near the end of the
+/// wave's region: a word past the row is read at the row's start, so that the two words of a read stay inside the region
+/// (the second is at most the one after the state row).
+struct RowBits
+{
+    i32 rel, keep;
+    u32 skip;
+};
+constexpr RowBits row_bits(const DevTerm& c, u32 w)
+{
+    const i32 rel = c.delta + 64 * static_cast<i32>(w), from = rel > 0 ? rel : 0, keep = static_cast<i32>(c.stride) - from;
+    return RowBits{rel, keep, static_cast<u32>(keep > 0 ? from : 0)};
+}
+
 /// One way an action changes a schema's successor count: its effect `effect` (position in the action's effect list),
 /// if the atom's bit changes, makes or unmakes the bindings whose literal is that atom. The literal's parameters are
 /// bound to the atom's objects (param[k] = term[k]: an action parameter, or -(object + 1)), the pairs eq must agree,
