@@ -417,6 +417,13 @@ void launch_dedup_rows(u64 start, u64 count, u32 words, u64 seed, double dup, u6
     launch_check("dedup rows");
 }
 
+/// hash_state of rows of no words.
+__global__ __launch_bounds__(kBlock) void k_hash_empty(u64 n, u64* __restrict__ out)
+{
+    for (u64 i = static_cast<u64>(blockIdx.x) * kBlock + threadIdx.x; i < n; i += static_cast<u64>(gridDim.x) * kBlock)
+        out[i] = mix64(kHashSeed);
+}
+
 /// Calls f.template operator()<W>() for a width of 1 to 16 words.
 template<u32 W = 1, class F>
 void with_narrow_width(u32 words, F&& f)
@@ -431,7 +438,9 @@ void launch_hash_rows(const u64* rows, u64 n, u32 words, u64* out, hipStream_t s
 {
     if (n == 0)
         return;
-    if (words > 16)
+    if (words == 0)
+        hipLaunchKernelGGL(k_hash_empty, dim3(static_cast<unsigned>(std::min<u64>(blocks_for(n, kBlock), 4096))), dim3(kBlock), 0, stream, n, out);
+    else if (words > 16)
         hipLaunchKernelGGL(k_hash_long, dim3(blocks_for(n, kHashWaves * kWave)), dim3(kHashWaves * kWave), 0, stream, rows, n, words, out);
     else
         with_narrow_width(words, [&]<u32 W>() {

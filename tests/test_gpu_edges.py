@@ -68,6 +68,20 @@ def test_hash_of_wide_rows(words, rows):
     assert [int(x) for x in got] == [port.hash_state(r) for r in a]
 
 
+@pytest.mark.parametrize("rows", [1, 64, 1000])
+def test_hash_of_rows_without_words(rows):
+    """The C ABI takes rows of no words: each hashes as the empty row."""
+    import torch
+
+    from mymyr_amd._lib import check, lib
+    from oracle import port
+
+    out = torch.zeros(rows, dtype=torch.int64, device="cuda")
+    check(lib.mya_hash_rows(out.data_ptr(), rows, 0, out.data_ptr(), None))
+    torch.cuda.synchronize()
+    assert [int(x) for x in out.cpu().numpy().view(np.uint64)] == [port.hash_state(np.zeros(0, np.uint64))] * rows
+
+
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("k", [1, 7, 40])
 def test_pad_of_rows_at_any_alignment(k, shift):
