@@ -62,11 +62,12 @@ TaskDev task_dev(const u64* img, const DevTaskHeader& h)
 
 namespace
 {
+constexpr size_t kCuLds = 160 * 1024;  // a CU's LDS, and the most a workgroup can have
+
 /// The waves per block that keep the most waves resident on a CU (its 160 KiB of LDS shared by whole blocks), for
 /// `wave` bytes per wave; a smaller block is taken only for at least 1/8 more resident waves.
 unsigned block_shape(size_t wave, size_t* lds_bytes)
 {
-    constexpr size_t kCuLds = 160 * 1024;
     constexpr int kCuWaves = 28;  // waves per CU the kernels' register use allows
     int nw = 1, best = 0;
     for (int k = kMaxWaves; k >= 1; --k)
@@ -591,9 +592,11 @@ void launch_expand(const ExpandArgs& args, hipStream_t stream)
     ExpandArgs a = args;
     a.wave_words = wave_words_of(a.wave_words, a.T, false);
     const bool simple = a.T.simple && !a.general;
-    // successors 64 at a time, where every instance is listable and the call asks for whole rows (rows narrower than the
-    // task's need their trimmed lengths, a successor at a time)
-    a.list = simple && a.T.listable && !a.unlistable && !a.witness && !a.succ_hash && (!a.succ || (!a.tasks && a.out_words >= a.T.W) || (a.tasks && a.out_words >= a.table_words));
+    // successors 64 at a time, where every instance is listable, the call asks for whole rows (rows narrower than the
+    // task's need their trimmed lengths, a successor at a time) and a workgroup has room for the list beside a wave's region
+    const u32 whole = a.tasks ? a.table_words : a.T.W;
+    a.list = simple && a.T.listable && !a.unlistable && !a.witness && !a.succ_hash && (!a.succ || a.out_words >= whole) &&
+             (u64{a.wave_words} + kListCap) * 8 <= kCuLds;
     size_t lds = 0;
     const unsigned nw = block_shape(static_cast<size_t>(a.wave_words + (a.list ? kListCap : 0)) * 8, &lds);
     if (a.witness && a.tasks)

@@ -54,8 +54,9 @@ constexpr u32 kMaxEff = 32;        // effects per schema the step applies (more 
 /// The word offsets of a wave's LDS region: the view, the state row, then the uniform binding, the 64 lanes' bindings
 /// (A = the largest schema arity, at least 1), the per-schema counts, for plans deeper than kLaneDepth the lanes'
 /// enumeration cursors (so far l_step words: the step's and the count's region), the successor enumeration's level
-/// cursors (A masks, A words) and its effect scratch. A step's region is what limits the waves of wide states: a
-/// transport_xl wave takes 22,824 bytes without the enumeration's scratch and 23,120 with it, seven waves to a CU or six
+/// cursors (A masks, A words) and its effect scratch. A read of two words at a bit position (row_bits) ends at most at
+/// the word after the row, the binding's. A step's region is what limits the waves of wide states: a
+/// transport_xl wave takes 22,816 bytes without the enumeration's scratch and 23,120 with it, seven waves to a CU or six
 /// (the allocation's granularity rounds the latter up past a seventh of the 160 KiB): 6.21 -> 5.38 ms per step.
 inline void set_region(TaskDev& t)
 {
@@ -71,11 +72,11 @@ inline void set_region(TaskDev& t)
     t.l_bind = next(32 * A);
     t.l_counts = next((t.num_schemas + 1) / 2);
     t.l_cur = next(A > kLaneDepth ? 64 * A + 32 * A : 0);
-    t.l_step = (w + 2) & ~1u;  // a word past the end: reads of two words at a bit position stay inside
+    t.l_step = (w + 1) & ~1u;
     t.l_dfs_m = next(A);
     t.l_dfs_w = next((A + 1) / 2);
     t.l_eff = next(kMaxEff / 2);
     t.l_before = next(kMaxEff / 2);
-    t.l_words = (w + 2) & ~1u;
+    t.l_words = (w + 1) & ~1u;
 }
 }  // namespace mya

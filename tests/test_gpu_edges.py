@@ -148,6 +148,36 @@ def test_expansion_equals_the_successor_listing(name, golden):
     assert torch.equal(d["succ"], x["succ"][keep]) and torch.equal(d["schema"], x["schema"][keep])
 
 
+def test_expansion_of_the_widest_rows():
+    """A state of 20,300 words leaves a wave's region in a workgroup's 160 KiB of LDS, but no room for the list of
+    bindings beside it: the expansion enumerates the successors one by one."""
+    import torch
+
+    from mymyr_amd import rl
+    from mymyr_amd.task import Task
+
+    n, preds, items = 64960, 20, 8
+    lines = [f"O {n}", f"P {preds + 2}", "S 1 item", *(f"F 1 p{k}" for k in range(preds)), "F 1 never", f"SI {items}",
+             *(f"0 {o}" for o in range(items)), "FI 1", "1 9", "G 1", "1 1 5", f"A {preds // 5 + 1}", "set 1", "L 2", "0 1 0", "1 0 0",
+             "E 1", "0", "L 0", "F 1", "1 1 0"]
+    for k in range(0, preds, 5):  # (every atom can be added, so every object has its slots; never applicable)
+        lines += [f"fill{k} 1", "L 1", f"{preds + 1} 1 0", "E 1", "0", "L 0", "F 5", *(f"{k + j + 1} 1 0" for j in range(5))]
+    t = Task.from_text("\n".join(lines) + "\n", "dense")
+    assert 20300 <= t.words <= 20316
+    s = torch.from_numpy(t.initial_state().view(np.int64).copy())[None].repeat(3, 1).cuda()
+    s[1, 0] |= 1 << 3
+    s[2, -1] |= 1
+    x = rl.expand(t, s, goal=True, hashes=True)
+    want = [(i, o) for i in range(3) for o in range(items) if not (int(s[i, 0]) >> o) & 1]
+    assert x["total"] == len(want) and x["binding"][:, 0].tolist() == [o for _, o in want]
+    for j, (i, o) in enumerate(want):
+        row = s[i].clone()
+        row[0] |= 1 << o
+        assert torch.equal(x["succ"][j], row) and int(x["goal"][j]) == (o == 5 or (int(s[i, 0]) >> 5) & 1)
+    count, _, binding, rows = rl.successors(t, s, cap=items)
+    assert count.tolist() == [8, 7, 8] and torch.equal(x["succ"][:8], rows[0])
+
+
 @pytest.mark.parametrize("words", [17, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257])
 def test_state_set_at_the_lane_group_shapes(words):
     """Rows at the edges of the probe's lane-group shapes, with duplicates inside a batch and across batches: ids are
