@@ -1664,7 +1664,7 @@ private:
             // bulk rows are read from the state itself: only the other pairs take view words
             p.offset = view_words;
             if (!p.bulk)
-                view_words += p.src_n * p.dst_words;
+                view_words = static_cast<u32>(std::min<u64>(u64{view_words} + u64{p.src_n} * p.dst_words, 0x7FFFFFFF));
             pairs.push_back(p);
         }
         // the terms of the steps' constraints, resolved against the pairs and the steps' windows
@@ -1750,11 +1750,10 @@ private:
                                         t.rows = p.src_n;
                             }
                         }
-                        // the wave's region holds the view, then the state row
+                        // the wave's region holds the view, then the state row (a region past 32-bit bit positions is far past
+                        // the LDS, so no launch reads such terms: the lifted kernels refuse the task, the ground search takes it)
                         const u64 bit0 = p.bulk ? 64 * static_cast<u64>(view_words) + p.bit0 : 64 * static_cast<u64>(p.offset);
                         const u64 row_bits = p.bulk ? p.row_bits : 64 * static_cast<u64>(p.dst_words);
-                        if (bit0 + row_bits * p.src_n > 0xFFFFFFFFull)
-                            throw Error("the task's state and view exceed the device path's 32-bit bit offsets");
                         if (row_bits % 64 == 0 && bit0 % 64 == 0 && delta >= 0 && delta % 64 == 0 && delta + 64 * static_cast<i64>(st.words) <= static_cast<i64>(row_bits))
                         {
                             t.path = static_cast<u32>(TermPath::Words);

@@ -258,3 +258,15 @@ def test_lazy_tasks_refused_by_env_tables(golden):
         rl.TaskTable([Task.from_text_file(golden.task_path("gripper__prob05")), t])
     with pytest.raises(MyaError, match="atoms must be"):
         _lib.check(lib.mya_task_load_file(golden.task_path("gripper__prob05").encode(), 4, ctypes.byref(h)))
+
+
+def test_tasks_whose_view_passes_32_bits_compile():
+    """Two binary fluents over the first and the last of 65,000 objects: their view rows span all objects (66 million words
+    each), past 32-bit bit positions. The lifted kernels cannot hold that, the ground search needs no view."""
+    n = 65000
+    lines = [f"O {n}", "P 4", "S 1 end", "F 2 a", "F 2 b", "F 0 z", "SI 2", "0 0", f"0 {n - 1}", "FI 1", f"1 0 {n - 1}", "G 1",
+             f"1 2 {n - 1} 0", "A 1", "flip 2", "L 4", "0 1 0", "0 1 1", "1 1 0 1", "2 0 0 1", "E 1", "0", "L 0", "F 3",
+             "1 0 0 1", "1 1 1 0", "2 1 1 0"]
+    for atoms in ("auto", "dense", "reachable"):
+        t = Task.from_text("\n".join(lines) + "\n", atoms)
+        assert t.words == 1 and t.label_width == 2
