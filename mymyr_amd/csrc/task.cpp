@@ -430,13 +430,15 @@ private:
         if (auto it = m_row_tables.find(key); it != m_row_tables.end())
             return it->second;
         const u32 id = static_cast<u32>(m_row_data.size());
-        Bits rows(static_cast<size_t>(std::max<u32>(n, 1)) * ow, 0);
+        Bits rows(static_cast<size_t>(std::max<u32>(n, 1)) * ow, 0), objects(ow, 0);
         for (const auto* a : static_atoms[pred])
         {
             const u32 f = (*a)[1 + from], t = (*a)[1 + to];
             rows[static_cast<size_t>(f) * ow + (t >> 6)] |= u64{1} << (t & 63);
+            set_bit(objects, t);
         }
         m_row_data.push_back(std::move(rows));
+        m_row_objects.push_back(std::move(objects));
         m_row_tables.emplace(key, id);
         return id;
     }
@@ -1669,10 +1671,12 @@ private:
         }
         // the terms of the steps' constraints, resolved against the pairs and the steps' windows
         std::vector<DevTerm> terms(cons.size());
-        std::vector<u64> term_rows;
-        std::vector<u8> static_term(cons.size(), 0);  // Image terms over term_rows (the others: over the dom0 bits)
+        // the rows of static relations cut to steps' windows: (row table, window start, words) -> first word; they are cut
+        // into the image itself (a large grid's rows are most of its image)
+        std::map<std::array<u32, 3>, u64> row_tables;
+        u64 term_row_words = 0;
+        std::vector<u8> static_term(cons.size(), 0);  // Image terms over those rows (the others: over the dom0 bits)
         {
-            std::map<std::array<u32, 3>, u32> row_tables;  // (static row table, window start, words) -> first word
             auto dom_bits = [&](u32 pred, u32 pos) {  // the objects an atom of `pred` can have at position `pos`
                 Bits b(ow, 0);
                 for (u32 o : C->layout.domain[C->layout.pos_begin[pred] + pos])
@@ -1700,30 +1704,15 @@ private:
                     Bits can(ow, 0);  // the objects the rows can hold
                     if (c.kind == static_cast<u32>(ConsKind::StaticRow))
                     {
-                        const std::vector<u64>& rows = m_row_data[c.table];
-                        for (u32 o = 0; o < n; ++o)
-                            for (u32 w = 0; w < ow; ++w)
-                                can[w] |= rows[static_cast<size_t>(o) * ow + w];
+                        can = m_row_objects[c.table];
                         const std::array<u32, 3> key{c.table, st.lo, st.words};
-                        auto it = row_tables.find(key);
-                        if (it == row_tables.end())
-                        {
-                            it = row_tables.emplace(key, static_cast<u32>(term_rows.size())).first;
-                            for (u32 o = 0; o < n; ++o)
-                                for (u32 w = 0; w < st.words; ++w)
-                                {
-                                    const u32 at = st.lo + 64 * w, sh = at & 63;
-                                    const u64* r = rows.data() + static_cast<size_t>(o) * ow;
-                                    u64 v = (at >> 6) < ow ? r[at >> 6] >> sh : 0;
-                                    if (sh && (at >> 6) + 1 < ow)
-                                        v |= r[(at >> 6) + 1] << (64 - sh);
-                                    term_rows.push_back(v);
-                                }
-                        }
+                        const auto [it, fresh] = row_tables.emplace(key, term_row_words);
+                        if (fresh)
+                            term_row_words += static_cast<u64>(n) * st.words;
                         t.path = static_cast<u32>(TermPath::Image);
                         static_term[ci] = 1;
                         t.src = c.src;
-                        t.base = it->second;
+                        t.base = static_cast<u32>(it->second);
                         t.stride = st.words;
                     }
                     else
@@ -1859,9 +1848,24 @@ private:
                 img.push_back(0);
         };
         const u64 off_dom0 = put(dom0_words.data(), dom0_words.size() * sizeof(u64));
-        const u64 off_term_rows = put(term_rows.data(), term_rows.size() * sizeof(u64));
-        if (img.size() > 0xFFFFFFF0ull)
+        if (img.size() + term_row_words > 0xFFFFFFF0ull)
             throw Error("the static relations' rows exceed the device image's 32-bit word offsets");
+        // (the sections that follow are small beside these; room for them, so that the image is not moved)
+        img.reserve(img.size() + term_row_words + C->layout.rs.size() * n + C->layout.fluent_count / 2 + 2 * records.size() + (u64{1} << 16));
+        const u64 off_term_rows = reserve_words(term_row_words);
+        for (const auto& [key, first] : row_tables)
+        {
+            const u64* r = m_row_data[key[0]].data();
+            u64* dst = img.data() + off_term_rows + first;
+            const u32 q = key[1] >> 6, sh = key[1] & 63, words = key[2];
+            for (u32 o = 0; o < n; ++o, r += ow, dst += words)
+            {
+                for (u32 w = 0; w < words && q + w < ow; ++w)
+                    dst[w] = r[q + w] >> sh;
+                for (u32 w = 0; sh && w < words && q + w + 1 < ow; ++w)
+                    dst[w] |= r[q + w + 1] << (64 - sh);
+            }
+        }
         align4();
         const u32 term0 = static_cast<u32>(img.size() / 4);
         for (size_t k = 0; k < terms.size(); ++k)
@@ -1996,6 +2000,7 @@ private:
     std::vector<Bits> s_unary;
     std::map<std::tuple<u32, u32, u32>, u32> m_row_tables;
     std::vector<Bits> m_row_data;
+    std::vector<Bits> m_row_objects;  // per row table: the objects its rows hold
     std::map<PairKey, u32> m_pairs;
     std::vector<PairKey> m_pair_list;
 };
