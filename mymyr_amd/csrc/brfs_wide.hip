@@ -551,7 +551,7 @@ BrfsResultC brfs_wide(const CompiledTask& task, const TaskDev& dev, const BrfsOp
                 if (layer_cut)
                 {
                     // the search goes on with the next layer: the cut winners' entries must not stand for states
-                    state_set_cut(set, cut_at, stream);
+                    state_set_cut(set, cut_at, size_dev, stream);
                     truncated = true;
                     break;
                 }

@@ -523,6 +523,7 @@ void state_set_clear(StateSet& s, hipStream_t stream)
     launch_check("clear state set");
     s.cur = 0;
     s.size = 0;
+    s.dead = 0;
     s.batches = 0;
     s.v.epoch = 0;
     s.last = stream;
@@ -530,7 +531,9 @@ void state_set_clear(StateSet& s, hipStream_t stream)
 
 void state_set_reserve(StateSet& s, u64 states, hipStream_t stream)
 {
-    if (s.v.capacity == s.slots || static_cast<double>(states) <= static_cast<double>(s.v.capacity) * s.max_load)
+    const bool whole = s.v.capacity == s.slots;
+    const double full = whole ? (1.0 + s.max_load) / 2 : s.max_load;
+    if ((whole && s.dead == 0) || static_cast<double>(states + s.dead) <= static_cast<double>(s.v.capacity) * full)
         return;
     s.v.capacity = s.slots;
     launch_fill_u32(reinterpret_cast<u32*>(s.v.table), s.v.capacity * 2, 0u, stream);
@@ -540,6 +543,7 @@ void state_set_reserve(StateSet& s, u64 states, hipStream_t stream)
         });
     launch_check("state set reserve");
     s.batches = 0;  // no entry holds an epoch
+    s.dead = 0;     // nor stands for no state
 }
 
 void state_set_begin_batch(StateSet& s, hipStream_t stream)
@@ -570,11 +574,12 @@ void state_set_resolve_ids(StateSet& s, const u64* cand_slot, u64 n, i64* ids, h
     launch_check("state set ids");
 }
 
-void state_set_cut(StateSet& s, u64 size, hipStream_t stream)
+void state_set_cut(StateSet& s, u64 size, u64 ranked, hipStream_t stream)
 {
     hipLaunchKernelGGL(k_cut_words, dim3(1), dim3(1), 0, stream, state_set_size_now(s), s.id_limit + s.v.epoch, size);
     launch_check("state set cut");
     s.size = size;
+    s.dead += ranked - size;
 }
 
 void state_set_probe(StateSet& s, const u64* rows, u64 m, hipStream_t stream, const BlockedView* blocked, u64* cand_slot)

@@ -43,6 +43,7 @@ struct StateSet
     u64 batches = 0;           // epochs taken since the last clear or settling pass
     u64 slots = 0;             // slots of the table's allocation (v.capacity: those in use)
     double max_load = 0;
+    u64 dead = 0;              // slots held by entries of no state (the winners past cuts)
 };
 
 /// Allocates a set for up to max_states rows of `words` words at the given maximum load: capacity =
@@ -51,8 +52,10 @@ struct StateSet
 /// the table's slots where they are a small part of it, and the driver calls state_set_reserve before each batch.
 void state_set_create(StateSet& s, u64 max_states, u32 words, double max_load, u64 batch_cap, hipStream_t stream,
                       u64 pending = 0, u64 start_slots = 0);
-/// Makes room for `states` stored and pending states on a set that started on part of its table: past the slots in use,
-/// the whole table is taken and the stored rows [0, s.size) (s.size must be exact, no batch under way) enter it anew.
+/// Makes room for `states` stored and pending states beside the dead entries of cuts: where a part of the table in use no
+/// longer holds them at the maximum load, the whole table is taken, and where dead entries fill the whole table (halfway
+/// from the maximum load to full, so that a pass follows a quarter of the slots' worth of cuts), it is cleared; the stored
+/// rows [0, s.size) (s.size must be exact, no batch under way) enter it anew.
 void state_set_reserve(StateSet& s, u64 states, hipStream_t stream);
 /// Frees the set's device memory: with a stream, in that stream's order (the blocks are reused only after the work
 /// queued on it so far, which must include every use of the set); without one, after the device has finished all work.
@@ -88,8 +91,9 @@ void state_set_rank(StateSet& s, u64 n, hipStream_t stream, u8* is_new = nullptr
 
 /// A cut inside the last ranked batch whose search goes on (a BrFS layer cut by max_next_layer_states): only the
 /// batch's winners below `size` are stored, so the set's size becomes `size` and the table entries of the others
-/// (pending codes of the batch's epoch) stand for no state from now on (the epoch's ids from `size` on are cut).
-void state_set_cut(StateSet& s, u64 size, hipStream_t stream);
+/// (pending codes of the batch's epoch) stand for no state from now on (the epoch's ids from `size` on are cut). `ranked`:
+/// the size with all of the batch's winners.
+void state_set_cut(StateSet& s, u64 size, u64 ranked, hipStream_t stream);
 
 /// The probe of a batch begun with state_set_begin_batch over candidate rows [m, words] (device) that the caller produced:
 /// a stored equal row drops a candidate, equal candidates keep the smallest index, the others take pending entries

@@ -242,3 +242,21 @@ def test_search_past_the_table_it_starts_on(props, max_states):
                                                                                       whole.fingerprint, whole.layer_counts)
     larger = search.brfs(task, **{**kw, "max_states": 1 << 25, "max_depth": len(whole.layer_counts) - 1})
     assert larger.layer_counts == whole.layer_counts[:-1]
+
+
+@pytest.mark.parametrize("limit, depth", [(500, 260), (3000, 160)])
+def test_layer_cuts_that_fill_the_table(limit, depth):
+    """Layers cut by max_next_layer_states leave the entries of the winners past the cut in the table, more in all than the
+    2^22 slots a search starts on and than the whole table of a search by small chunks, while few states are stored. The
+    table is taken whole, or cleared and its states entered anew: the same search however large it is."""
+    from mymyr_amd import gen, search
+    from mymyr_amd.task import Task
+
+    task = Task.from_text(gen.random_strips(512, 4096, init_atoms=64, seed=4), "dense")
+    kw = dict(max_depth=depth, max_states=limit * depth + 100000, max_next_layer_states=limit, layer_order="in_order", stop_at_goal=False,
+              fingerprint=True)
+    runs = [search.brfs(task, **kw, **c) for c in ({}, {"chunk": 1 << 21}, {"chunk": 1 << 17}, {"chunk": 1 << 23})]
+    assert runs[0].layers == depth and all(new == limit for _, _, new in runs[0].layer_counts[-depth // 2:])
+    for r in runs[1:]:
+        assert (r.states, r.expanded, r.generated, r.fingerprint, r.layer_counts) == (runs[0].states, runs[0].expanded, runs[0].generated,
+                                                                                      runs[0].fingerprint, runs[0].layer_counts)
