@@ -399,8 +399,8 @@ class BatchedEnv:
     def set_launch(self, launch: str) -> None:
         """'widest' or 'per_bucket' (BatchedEnv.set_launch, python/mymyr/rl/torch/_batched.py:573-575): how the
         reference's device env launches over a table's row-width buckets. The HIP env picks its launch shape itself
-        (rows grouped by instance on the device, one launch per instance of a table of at most 16 instances, else one
-        per kernel variant); the outputs do not depend on it, so either value is accepted and recorded."""
+        (one launch in batch order, each row with its own instance's tables); the outputs do not depend on it, so either
+        value is accepted and recorded."""
         if launch not in ("widest", "per_bucket"):
             raise ValueError("mymyr: launch must be 'widest' or 'per_bucket'")
         self.launch = launch

@@ -192,8 +192,8 @@ ExpandScratch carve_expand_scratch(void* block, u64 n)
     return x;
 }
 
-/// The flat expansion of rows over instances `inst` (several: `env`'s, with the rows' task ids). `block` (device, at least expand_scratch_bytes(max(rows, 1)) bytes) holds the
-/// expansion's scratch; the call synchronizes the stream before it returns, so the block is free again then.
+/// The flat expansion of rows over instances `inst` (several: `env`'s, with the rows' task ids). `block` (device, at least
+/// expand_scratch_bytes(max(rows, 1)) bytes) holds the expansion's scratch; the call synchronizes the stream before it returns, so the block is free again then.
 void expand_rows(const std::vector<const TaskDev*>& inst, mya_env* env, const int32_t* task_ids, const uint64_t* states, uint64_t rows,
                  uint32_t words, const mya_expand_options* options, mya_expansion* out, hipStream_t stream, void* block, mya_task* lazy)
 {

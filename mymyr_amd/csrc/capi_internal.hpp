@@ -100,7 +100,7 @@ constexpr size_t expand_scratch_bytes(u64 n)
 ExpandScratch carve_expand_scratch(void* block, u64 n);
 
 /// The flat expansion of rows over instances `inst` (several: `env`'s
-/// scratch and the rows' task ids). `block` (device, at least expand_scratch_bytes(max(rows, 1)) bytes) holds the
+/// tables and the rows' task ids). `block` (device, at least expand_scratch_bytes(max(rows, 1)) bytes) holds the
 /// expansion's scratch; the call synchronizes the stream before it returns, so the block is free again then.
 /// `lazy`: the one instance's task when it has lazy slots (its atoms are interned between repeats of the successor
 /// pass; the caller holds its lazy_mutex), else null.

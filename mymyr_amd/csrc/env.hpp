@@ -1,8 +1,8 @@
 #pragma once
 // The batched environment step on the device, bit-exact with HostEnv::step_row_impl (src/mymyr/rl/env.cpp:351-528):
 // choose (given index or Philox draw over the canonical successor order), move, goal, dead end, reward, termination,
-// truncation, successor count of the reached state, SAME_STEP autoreset. One wavefront per environment row, several
-// waves per block sharing the LDS copy of the task's hot tables.
+// truncation, successor count of the reached state, SAME_STEP autoreset. One wavefront per environment row, with the
+// row and its view in the wave's own LDS region and the task's tables read through the caches.
 
 #include "lifted.hpp"
 

@@ -107,7 +107,7 @@ void state_set_probe(StateSet& s, const u64* rows, u64 m, hipStream_t stream, co
 /// entries are not read by callers).
 void state_set_resolve_ids(StateSet& s, const u64* cand_slot, u64 n, i64* ids, hipStream_t stream);
 
-/// hash_state of every row (a group of lanes per row).
+/// hash_state of every row (a lane per row).
 void launch_hash_rows(const u64* rows, u64 n, u32 words, u64* out, hipStream_t stream);
 
 /// Fills n u32 words with v.
