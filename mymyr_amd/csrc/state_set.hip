@@ -81,15 +81,18 @@ __global__ __launch_bounds__(kBlock) void k_hash_narrow(const u64* __restrict__ 
         out[first + lane] = mix64(h);
 }
 
-/// hash_state of rows above 16 words, a lane per row as k_hash_narrow: 64 rows' chains run side by side, and the wave reads
-/// the rows 16 words at a time through LDS (whole 128-byte lines, rows padded to 17 words so that the lanes' reads of one
-/// word fall on different banks). The chain starts from the trimmed length, found from the rows' last tiles first. Bound
-/// by the reads: 4.0 TB/s on the 176-word successors of 8,195 transport states.
+/// hash_state of many rows above 16 words, a lane per row as k_hash_narrow: 64 rows' chains run side by side, and the wave
+/// reads the rows 16 words at a time through LDS (whole 128-byte lines, rows padded to 17 words so that the lanes' reads of
+/// one word fall on different banks). The chain starts from the trimmed length, found from the rows' last tiles first. Many
+/// rows are bound by the reads: 4.0 TB/s on the 176-word successors of 8,195 transport states. Some thousand rows are
+/// bound by the chain (100 ns a word pair), so while one tile is hashed the next comes from LDS and the one after it from
+/// memory: 4,096 rows of 1,024 words 93 us with a tile's latencies between the folds, 63 us so.
 constexpr u32 kHashTile = 16;
 constexpr int kHashWaves = 4;
 __global__ __launch_bounds__(kHashWaves * kWave) void k_hash_long(const u64* __restrict__ rows, u64 n, u32 words, u64* __restrict__ out)
 {
     __shared__ u64 tiles[kHashWaves][kWave * (kHashTile + 1)];
+    constexpr u32 kStep = kWave / kHashTile;  // rows that the lanes read side by side
     const u32 lane = lane_id(), wave = threadIdx.x / kWave;
     u64* tile = tiles[wave];
     const u64* mine = tile + lane * (kHashTile + 1);
@@ -98,45 +101,145 @@ __global__ __launch_bounds__(kHashWaves * kWave) void k_hash_long(const u64* __r
         return;  // whole waves: barriers below are wave-wide
     const u32 count = static_cast<u32>(min(static_cast<u64>(kWave), n - first));
     const u32 last = (words - 1) / kHashTile;
+    const u32 c = lane % kHashTile, r0 = lane / kHashTile;
     // words [16 t, 16 t + 16) of the wave's rows (zeros past the rows' words): lanes 16 r + c take word c of row 4 k + r
-    auto load = [&](u32 t) {
-        const u32 c = lane % kHashTile, w = t * kHashTile + c;
-        u64 v[kHashTile];
+    auto fetch = [&](u32 t, u64 (&v)[kHashTile]) {
+        const u32 w = t * kHashTile + c;
+        const u64* src = rows + (first + r0) * words + w;
 #pragma unroll
         for (u32 k = 0; k < kHashTile; ++k)
-        {
-            const u32 r = k * (kWave / kHashTile) + lane / kHashTile;
-            v[k] = r < count && w < words ? rows[(first + r) * words + w] : 0;
-        }
+            v[k] = k * kStep + r0 < count && w < words ? src[static_cast<u64>(k * kStep) * words] : 0;
+    };
+    // the fetched words to the lanes of their rows
+    auto hand = [&](const u64 (&v)[kHashTile]) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
         for (u32 k = 0; k < kHashTile; ++k)
-            tile[(k * (kWave / kHashTile) + lane / kHashTile) * (kHashTile + 1) + c] = v[k];
+            tile[(k * kStep + r0) * (kHashTile + 1) + c] = v[k];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    u32 len = 0;  // 1 + the highest nonzero word
-    for (u32 t = last + 1; t > 0 && __ballot(len == 0 && lane < count); --t)
-    {
-        load(t - 1);
-        for (u32 c = 0; c < kHashTile; ++c)
-            if (mine[c] && len < (t - 1) * kHashTile + c + 1 && (len == 0 || len > (t - 1) * kHashTile))
-                len = (t - 1) * kHashTile + c + 1;
-    }
-    u64 h = kHashSeed ^ (static_cast<u64>(len) * kHashP1);
-    for (u32 t = 0; __ballot(t * kHashTile < len); ++t)
-    {
-        load(t);
+    auto take = [&](u64 (&x)[kHashTile]) {
 #pragma unroll
-        for (u32 c = 0; c < kHashTile; c += 2)
-            if (t * kHashTile + c < len)
-                h = mulfold(h ^ mine[c] ^ kHashP1, mine[c + 1] ^ kHashP2);
+        for (u32 q = 0; q < kHashTile; ++q)
+            x[q] = mine[q];
+    };
+    u64 a[kHashTile], x[kHashTile], y[kHashTile];
+    u32 len = 0;  // 1 + the highest nonzero word
+    fetch(last, x);
+    fetch(0, a);
+    for (u32 t = last;; --t)
+    {
+        hand(x);
+        if (t && t != last)
+            fetch(t - 1, x);  // (a second tile is rarely needed, a third follows it often)
+        const bool open = len == 0;
+#pragma unroll
+        for (u32 q = 0; q < kHashTile; ++q)
+            len = open && mine[q] ? t * kHashTile + q + 1 : len;
+        if (t == 0 || !__ballot(len == 0 && lane < count))
+            break;
+        if (t == last)
+            fetch(t - 1, x);
+    }
+    const u32 end = (group_max<kWave>(len) + kHashTile - 1) / kHashTile;
+    u64 h = kHashSeed ^ (static_cast<u64>(len) * kHashP1);
+    // while tile t is hashed from x, tile t + 1 comes from LDS into y and tile t + 2 from memory
+    auto step = [&](u32 t, const u64 (&cur)[kHashTile], u64 (&next)[kHashTile]) {
+        if (t + 1 < end)
+        {
+            hand(a);
+            take(next);
+            if (t + 2 < end)
+                fetch(t + 2, a);
+        }
+        if (!__ballot(lane < count && len < (t + 1) * kHashTile))
+        {
+            // every row goes on past the tile: nothing but the multiply-folds on the chain
+#pragma unroll
+            for (u32 q = 0; q < kHashTile; q += 2)
+                h = mulfold(h ^ (cur[q] ^ kHashP1), cur[q + 1] ^ kHashP2);
+            return;
+        }
+#pragma unroll
+        for (u32 q = 0; q < kHashTile; q += 2)
+        {
+            const u64 folded = mulfold(h ^ (cur[q] ^ kHashP1), cur[q + 1] ^ kHashP2);
+            h = t * kHashTile + q < len ? folded : h;
+        }
+    };
+    hand(a);
+    take(x);
+    if (end > 1)
+        fetch(1, a);
+    for (u32 t = 0; t < end; t += 2)
+    {
+        step(t, x, y);
+        if (t + 1 < end)
+            step(t + 1, y, x);
     }
     if (lane < count)
         out[first + lane] = mix64(h);
+}
+
+/// hash_state of few rows above 16 words, a wave per row: the lanes read 64 word pairs side by side and the chain runs on
+/// the scalar unit, whose multiplies return sooner than the vector unit's (60 ns a pair against 100). One row of 2,048 words
+/// 62 us, against 107 by k_hash_long.
+__global__ __launch_bounds__(kBlock) void k_hash_wave(const u64* __restrict__ rows, u64 n, u32 words, u64* __restrict__ out)
+{
+    const u32 lane = lane_id();
+    const u32 wave = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave)));
+    const u64 j = static_cast<u64>(blockIdx.x) * (kBlock / kWave) + wave;
+    if (j >= n)
+        return;
+    const u64* row = rows + j * words;
+    // pairs [64 t, 64 t + 64) of the row, one per lane (zeros past its words)
+    auto fetch = [&](u32 t, u64& lo, u64& hi) {
+        const u32 w = 2 * (t * kWave + lane);
+        lo = w < words ? row[w] : 0;
+        hi = w + 1 < words ? row[w + 1] : 0;
+    };
+    u64 lo, hi, nz;
+    u32 t = (words - 1) / (2 * kWave);
+    for (;; --t)
+    {
+        fetch(t, lo, hi);
+        nz = __ballot((lo | hi) != 0);
+        if (nz || t == 0)
+            break;
+    }
+    u32 len = 0;  // 1 + the highest nonzero word
+    if (nz)
+    {
+        const u32 top = kWave - 1 - static_cast<u32>(__builtin_clzll(nz));
+        len = 2 * (t * kWave + top) + (lane_value(hi, top) ? 2 : 1);
+    }
+    u64 h = kHashSeed ^ (static_cast<u64>(len) * kHashP1);
+    const u32 pairs = (len + 1) / 2;
+    fetch(0, lo, hi);
+    for (u32 p = 0; p < pairs; p += kWave)
+    {
+        u64 next_lo = 0, next_hi = 0;
+        if (p + kWave < pairs)
+            fetch(p / kWave + 1, next_lo, next_hi);
+        auto fold = [&](u32 k) { h = mulfold(h ^ lane_value(lo, k) ^ kHashP1, lane_value(hi, k) ^ kHashP2); };
+        if (pairs - p >= kWave)
+        {
+#pragma unroll
+            for (u32 k = 0; k < kWave; ++k)
+                fold(k);
+        }
+        else
+            for (u32 k = 0; k < pairs - p; ++k)
+                fold(k);
+        lo = next_lo;
+        hi = next_hi;
+    }
+    if (lane == 0)
+        out[j] = mix64(h);
 }
 
 template<int G, int K>
@@ -434,12 +537,18 @@ void with_narrow_width(u32 words, F&& f)
         with_narrow_width<W + 1>(words, f);
 }
 
+/// At most this many rows above 16 words are hashed a wave each, more a lane each: two waves for each of the chip's 1,024
+/// SIMDs still run side by side (2,048 rows of 1,024 words: 51 us by waves, 64 by lanes; 4,096 rows: 90 and 63).
+constexpr u64 kWaveHashRows = 2048;
+
 void launch_hash_rows(const u64* rows, u64 n, u32 words, u64* out, hipStream_t stream)
 {
     if (n == 0)
         return;
     if (words == 0)
         hipLaunchKernelGGL(k_hash_empty, dim3(static_cast<unsigned>(std::min<u64>(blocks_for(n, kBlock), 4096))), dim3(kBlock), 0, stream, n, out);
+    else if (words > 16 && n <= kWaveHashRows)
+        hipLaunchKernelGGL(k_hash_wave, dim3(blocks_for(n, kBlock / kWave)), dim3(kBlock), 0, stream, rows, n, words, out);
     else if (words > 16)
         hipLaunchKernelGGL(k_hash_long, dim3(blocks_for(n, kHashWaves * kWave)), dim3(kHashWaves * kWave), 0, stream, rows, n, words, out);
     else

@@ -68,6 +68,26 @@ def test_hash_of_wide_rows(words, rows):
     assert [int(x) for x in got] == [port.hash_state(r) for r in a]
 
 
+@pytest.mark.parametrize("words", [17, 33, 127, 128, 129, 176, 300])
+@pytest.mark.parametrize("rows", [3, 2048, 2049, 2100])
+def test_hash_of_few_and_many_wide_rows(words, rows):
+    """Rows above 16 words hashed a wave each (up to 2,048) and a lane each: rows around the line, widths around the 128
+    words that a wave reads at once, trimmed lengths of no tile to all, whole waves of short rows."""
+    import torch
+
+    from mymyr_amd import hip
+    from oracle import port
+
+    rng = np.random.default_rng(words * 1000 + rows)
+    a = rng.integers(0, 1 << 63, size=(rows, words), dtype=np.uint64)
+    for i in range(0, rows, 3):
+        a[i, rng.integers(0, words + 1):] = 0
+    a[64:128, 5:] = 0
+    a[0] = 0
+    got = hip.hash_rows(torch.from_numpy(a.view(np.int64)).cuda()).cpu().numpy().view(np.uint64)
+    assert [int(x) for x in got] == [port.hash_state(r) for r in a]
+
+
 @pytest.mark.parametrize("rows", [1, 64, 1000])
 def test_hash_of_rows_without_words(rows):
     """The C ABI takes rows of no words: each hashes as the empty row."""
