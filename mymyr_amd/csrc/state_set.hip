@@ -448,18 +448,21 @@ void with_shape(u32 W, F&& f)
         f.template operator()<4, 1>();
     else if (W <= 16)
         f.template operator()<4, 2>();  // four lanes of two pairs: faster than eight of one on 16-word rows
-    // sixteen lanes a row up to 256 words: four rows' probe chains (row, entry, compared row) in flight per wave where a
-    // wave per row waits for one (transport search, 176-word rows)
+    // sixteen lanes a row up to 192 words: four rows' probe chains (row, entry, compared row) in flight per wave where a
+    // wave per row waits for one (131,072 rows of 176 words 122 -> 108 us); above, the four rows' words take the registers
+    // of the waves that would hide their latency (of 256 words 141 us by a wave, 176 by sixteen lanes of eight pairs)
     else if (W <= 32)
         f.template operator()<16, 1>();
     else if (W <= 64)
         f.template operator()<16, 2>();
     else if (W <= 128)
         f.template operator()<16, 4>();
+    else if (W <= 160)
+        f.template operator()<16, 5>();
     else if (W <= 192)
         f.template operator()<16, 6>();
     else if (W <= 256)
-        f.template operator()<16, 8>();
+        f.template operator()<64, 2>();
     else if (W <= 512)
         f.template operator()<64, 4>();
     else if (W <= 1024)

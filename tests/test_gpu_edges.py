@@ -198,7 +198,7 @@ def test_expansion_of_the_widest_rows():
     assert count.tolist() == [8, 7, 8] and torch.equal(x["succ"][:8], rows[0])
 
 
-@pytest.mark.parametrize("words", [17, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257])
+@pytest.mark.parametrize("words", [17, 32, 33, 64, 65, 128, 129, 160, 161, 192, 193, 256, 257])
 def test_state_set_at_the_lane_group_shapes(words):
     """Rows at the edges of the probe's lane-group shapes, with duplicates inside a batch and across batches: ids are
     first-occurrence ranks."""
