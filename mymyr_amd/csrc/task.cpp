@@ -1477,8 +1477,12 @@ private:
         // object: a constant, or a parameter's static domain). No such effect: the count stays. Where the effects of one
         // sign meet at most one literal of s, a positive one, the bindings lost are those of the state whose literal is
         // a deleted atom and the bindings gained those of the reached state whose literal is an added atom (DevDelta);
-        // otherwise, and with more than 32 schemas, s is counted again.
+        // otherwise, and with more than 32 schemas, s is counted again. Tasks that are not simple have small relations and
+        // many schemas: there two deltas of a schema wait longer for their records, tests and plans than one count of it
+        // does, so s is counted again from two matches on (rovers, 9 schemas: 64 envs 111 -> 95 us a step, 8,192 envs
+        // 233 -> 188; freecell 89 -> 80 and 194 -> 171; none of ten such tasks slower).
         {
+            const bool simple = checks.empty() && C->label_width <= kLaneDepth + 1;
             const u32 S = static_cast<u32>(schemas.size());
             auto dom_of = [&](u32 si, i32 t) {
                 Bits b(ow, 0);
@@ -1603,7 +1607,7 @@ private:
                         }
                     if (matches.empty())
                         continue;
-                    plain = plain && lits[0].size() <= 1 && lits[1].size() <= 1 && matches.size() <= 8;
+                    plain = plain && lits[0].size() <= 1 && lits[1].size() <= 1 && matches.size() <= (simple ? 8u : 1u);
                     std::vector<DevDelta> mine;
                     for (const Match& m : matches)
                     {
