@@ -1854,8 +1854,9 @@ private:
         const u64 off_dom0 = put(dom0_words.data(), dom0_words.size() * sizeof(u64));
         if (img.size() + term_row_words > 0xFFFFFFF0ull)
             throw Error("the static relations' rows exceed the device image's 32-bit word offsets");
-        // (the sections that follow are small beside these; room for them, so that the image is not moved)
-        img.reserve(img.size() + term_row_words + C->layout.rs.size() * n + C->layout.fluent_count / 2 + 2 * records.size() + (u64{1} << 16));
+        // where these are most of the image, room for the sections that follow, so that it is not moved
+        if (term_row_words >= u64{1} << 16)
+            img.reserve(img.size() + term_row_words + C->layout.rs.size() * n + C->layout.fluent_count / 2 + 2 * records.size() + (u64{1} << 16));
         const u64 off_term_rows = reserve_words(term_row_words);
         for (const auto& [key, first] : row_tables)
         {
