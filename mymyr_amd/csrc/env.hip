@@ -68,7 +68,9 @@ constexpr size_t kCuLds = 160 * 1024;  // a CU's LDS, and the most a workgroup c
 /// `wave` bytes per wave; a smaller block is taken only for at least 1/8 more resident waves.
 unsigned block_shape(size_t wave, size_t* lds_bytes)
 {
-    constexpr int kCuWaves = 28;  // waves per CU the kernels' register use allows
+    // the waves per CU that the registers of the simple tasks' steps and counts allow; of their expansions 24 and of the
+    // general kernels 20 are resident, and the shape chosen against 28 holds as many of them as one chosen against these
+    constexpr int kCuWaves = 28;
     int nw = 1, best = 0;
     for (int k = kMaxWaves; k >= 1; --k)
     {

@@ -122,18 +122,10 @@ __device__ __forceinline__ Lds lds_of(lds<u64>* region, const TaskDev& T)
     return l;
 }
 
-/// The same record behind a pointer the compiler knows nothing about: loads through it are made where they are used.
-/// The kernels have more invariant fields (arguments, table pointers, LDS offsets) than scalar registers, and hoisted to
-/// the kernel's start they spill into vector lanes (900 spills in the step, a third of its vector instructions); a
-/// scalar load again is one cached access.
-template<class X>
-__device__ __forceinline__ const X& fresh(const X& x)
-{
-    cst<X>* p = (cst<X>*)&x;
-    asm volatile("" : "+s"(p));
-    return *(const X*)p;
-}
-/// The kernel's argument record (its first argument), as fresh.
+/// The kernel's argument record (its first argument) behind a pointer the compiler knows nothing about: loads through it
+/// are made where they are used. The kernels have more invariant fields (arguments, table pointers, LDS offsets) than
+/// scalar registers, and hoisted to the kernel's start they spill into vector lanes (900 spills in the step, a third of
+/// its vector instructions); a scalar load again is one cached access.
 template<class X>
 __device__ __forceinline__ const X& kernel_args()
 {

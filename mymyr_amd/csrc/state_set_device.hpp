@@ -206,45 +206,35 @@ __device__ __forceinline__ bool group_equal(const Slice<G, K>& a, const Slice<G,
     return group_all<G>(eq, gbase);
 }
 
-/// hash_state of the group's row (group-uniform).
+/// hash_state of the group's row (group-uniform), for the narrow rows that are placed by it (group_set_hash).
 template<int G, int K>
 __device__ __forceinline__ u64 group_hash(const Slice<G, K>& s, u32 q, u32 gbase)
 {
-    if constexpr (K == 0)
-    {
-        // the serial chain of hash_state over the trimmed words, on the group's first lane
-        u64 h = 0;
-        if (q == 0)
-            h = hash_state(s.row, s.W);
-        return group_bcast<G>(h, gbase, 0);
-    }
-    else
-    {
-        u32 top = 0;  // 1 + index of the lane's highest nonzero word
+    static_assert(K > 0, "rows in registers");
+    u32 top = 0;  // 1 + index of the lane's highest nonzero word
 #pragma unroll
-        for (int k = 0; k < K; ++k)
+    for (int k = 0; k < K; ++k)
+    {
+        const u32 w = 2 * (k * G + q);
+        if (s.hi[k])
+            top = w + 2;
+        else if (s.lo[k])
+            top = w + 1;
+    }
+    const u32 n = group_max<G>(top);
+    u64 h = kHashSeed ^ (static_cast<u64>(n) * kHashP1);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int r = 0; r < G; ++r)
         {
-            const u32 w = 2 * (k * G + q);
-            if (s.hi[k])
-                top = w + 2;
-            else if (s.lo[k])
-                top = w + 1;
+            const u32 p = k * G + r;
+            const u64 a = group_bcast<G>(s.lo[k], gbase, r);
+            const u64 b = group_bcast<G>(s.hi[k], gbase, r);
+            if (2 * p < n)
+                h = mulfold(h ^ a ^ kHashP1, b ^ kHashP2);
         }
-        const u32 n = group_max<G>(top);
-        u64 h = kHashSeed ^ (static_cast<u64>(n) * kHashP1);
-#pragma unroll
-        for (int k = 0; k < K; ++k)
-#pragma unroll
-            for (int r = 0; r < G; ++r)
-            {
-                const u32 p = k * G + r;
-                const u64 a = group_bcast<G>(s.lo[k], gbase, r);
-                const u64 b = group_bcast<G>(s.hi[k], gbase, r);
-                if (2 * p < n)
-                    h = mulfold(h ^ a ^ kHashP1, b ^ kHashP2);
-            }
-        return mix64(h);
-    }
+    return mix64(h);
 }
 
 /// Rows wider than this many words are placed in the table by set_hash_wide instead of hash_state.
