@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kTW * kWave) void k_ground_emit(const u64* __restri
 // offsets and total, the first goal state and the goal states' number, the chunk's end (as k_chunk_end) and the set's size and
 // status into the driver's scalars. Launch by launch (three of the scan, the goal search's two, the
 // chunk's end, the gather and the copy) a layer of 10^4 parents spends longer in the gaps than in the kernels: all of a
-// gripper task, 26 such layers, 3.49 -> 2.25 ms with these in one. Each thread has its counts of all passes in flight at
+// gripper task, 26 such layers, 3.6 -> 2.2 ms with these in one. Each thread has its counts of all passes in flight at
 // once; a pass is 4,096 parents, four to a thread.
 constexpr u32 kLayerPasses = 8;
 constexpr u32 kLayerPass = 4 * 1024;
@@ -712,10 +712,10 @@ __global__ __launch_bounds__(kLB) void k_ground_compact(StateSetView s, ParentRo
 // probes, ranks and rows. Its winners' entries are settled to their ids on the spot, so the layers share one epoch. A layer
 // that is not all plain is left untouched for the host's path: more than kSmallParents parents or kSmallLanes lanes of
 // successors, the expansion budget ending inside it, or successors that could fill the store. A goal state to stop at
-// ends the search here, its layer expanded up to it (a layer on the host's path less: 0.77 -> 0.58 ms of a shortest path).
+// ends the search here, its layer expanded up to it (a layer on the host's path less: 0.79 -> 0.68 ms of a shortest path).
 //
-// Shortest path in a 32x32 grid (16 layers, 16-word rows) 2.69 -> 1.05 ms, all of a gripper task (36 layers, the smaller of
-// them here) 5.54 -> 3.89 ms, both with the plan's records read at once (plan_nodes); a search whose layers explode is as
+// Shortest paths in a 32x32 grid (mean of six start states, some 20 layers, 16-word rows) 3.35 -> 1.10 ms, all of a gripper task (36 layers, the smaller of
+// them here) 5.6 -> 3.9 ms, both with the plan's records read at once (plan_nodes); a search whose layers explode is as
 // before. The limit on lanes is eight rounds of probes of the block's threads.
 constexpr u32 kSmallThreads = 1024;
 constexpr u32 kSmallWaves = kSmallThreads / kWave;
