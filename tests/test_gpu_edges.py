@@ -52,8 +52,8 @@ def test_counts_after_a_move_equal_a_recount(name, golden):
 @pytest.mark.parametrize("words", [*range(1, 17), 17, 18, 31, 32, 33, 47, 176, 200, 1025])
 @pytest.mark.parametrize("rows", [1, 63, 64, 65, 257])
 def test_hash_of_wide_rows(words, rows):
-    """Rows hashed by a lane each, 64 to a wave and 16 words at a time: row counts around a wave, widths around a tile,
-    rows whose trimmed length ends anywhere (an empty row included)."""
+    """Rows up to 16 words hashed by a lane each, 64 to a wave, and these few wider ones by a wave each: row counts around a
+    wave, widths around a tile, rows whose trimmed length ends anywhere (an empty row included)."""
     import torch
 
     from mymyr_amd import hip
